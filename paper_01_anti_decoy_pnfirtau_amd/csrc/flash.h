@@ -23,6 +23,7 @@ struct FwdParams {
   // causal FIR taps ([fir_taps_rows][fir_k] fp32, as pnfx_fir_fwd) before its scores
   const float* fir_taps = nullptr;
   int fir_taps_rows = 0, fir_k = 0;
+  int grp = 2;  // bf16: (b, h) slices per dispatch group (slice_group)
 };
 
 struct BwdParams {
@@ -45,7 +46,19 @@ struct BwdParams {
   int B, H, N, nq32, nk64, nkvb;
   const float* tau;
   float scale, gamma;
+  int grp = 2;  // bf16: (b, h) slices per dispatch group (slice_group)
 };
+
+// (b, h) slices per dispatch group of the bf16 kernels: as many as keep the group's streamed pair of
+// operands (N rows of 4 D bytes a slice) within one XCD's 4 MiB of L2, at least two.  Larger groups
+// dispatch more heavy causal blocks first, so fewer run alone at the end; groups past the L2 re-read
+// their tiles from beyond it (at B=4 H=16 N=8192 d=64, two slices, groups of four took 2-3x the
+// misses for nothing in the gradients).  With half the key tiles silent at B=4 H=16 N=4096 d=64, groups
+// of four instead of two: dK/dV 258 -> 213 us, forward 130 -> 125.
+inline int slice_group(int64_t N, int64_t D) {
+  const int64_t g = (4ll << 20) / (N * D * 4);
+  return (int)(g < 2 ? 2 : g > 64 ? 64 : g);
+}
 
 // 16-row MFMA query blocks per wave of the bf16 dQ kernel (workgroups of four waves cover
 // 64 * dq_qblocks(D) query rows).

@@ -225,24 +225,43 @@ __device__ __forceinline__ float pow10f_(float u) {
 }
 
 // Map a linear block id to (bh, block index).  Each XCD (block id % 8 on the round-robin
-// dispatcher) works through a contiguous range of (b, h) slices, so their K/V (forward, dQ)
-// or Q/dO (dK/dV) tiles stay in that XCD's L2.  Within the range, slices go in pairs, and a
-// pair's blocks are dispatched heaviest first across both slices: causal blocks range from
-// one tile of work to N/64, and ordering them one slice at a time leaves the last slice's
-// heavy blocks to start late and run alone.  Measured at C4 against one slice at a time:
-// forward -3 %, dQ -4 %, dK/dV -2 % (-9 % with silent key tiles), for 20-25 % more L2
-// misses; groups of four gain another 1-3 % on the forward only, at 2-3x the misses.
-__device__ __forceinline__ void map_block(int nblk, int BH, bool heavy_last_index, int& bh,
+// dispatcher) owns BH / 8 whole (b, h) slices, so their K/V (forward, dQ) or Q/dO (dK/dV) tiles
+// stay in that XCD's L2; the blocks of the BH % 8 slices left over are dealt to all XCDs in turn,
+// mixed evenly among the owned ones.  Own slices go in groups of `grp`, and a group's blocks are
+// dispatched heaviest first across its slices: causal blocks range from one tile of work to N/64,
+// and in smaller groups the last group's heavy blocks start late and run alone.  See slice_group
+// for the size of the groups.
+__device__ __forceinline__ void map_block(int nblk, int BH, int grp, bool heavy_last_index, int& bh,
                                           int& blk) {
-  constexpr int G = 2;
-  const int total = nblk * BH;
-  int L = blockIdx.x;
-  if ((total & 7) == 0) L = (L & 7) * (total >> 3) + (L >> 3);
-  const int c = L / (G * nblk), r = L % (G * nblk);
-  const int ge = min(G, BH - c * G);  // the last group may hold fewer slices
-  bh = c * G + r % ge;
-  const int j = r / ge;
-  blk = heavy_last_index ? nblk - 1 - j : j;
+  const unsigned xcd = blockIdx.x & 7, own = (unsigned)BH >> 3, left = (unsigned)BH & 7;
+  unsigned r = blockIdx.x >> 3;  // the XCD's r-th workgroup
+  unsigned first = xcd * own, ge = own;
+  bool dealt = false;
+  if (left) {
+    // The XCD's sequence mixes its n_own own blocks with the n_left dealt to it: p0 own ones come
+    // before its i-th workgroup.
+    const unsigned i = r, n_own = own * nblk, n_left = (left * nblk - xcd + 7) >> 3;
+    const auto own_before = [&](unsigned k) {
+      const unsigned m = min(k - k * left / (unsigned)BH, n_own);
+      return k > n_left ? max(m, k - n_left) : m;
+    };
+    r = own_before(i);
+    if (own_before(i + 1) == r) {
+      dealt = true;
+      r = (i - r) * 8 + xcd;  // index among all the dealt blocks
+      first = 8 * own;
+      ge = left;
+    }
+  }
+  if (!dealt && (unsigned)grp < own) {  // own slices in groups (the last may hold fewer)
+    const unsigned c = r / (unsigned)(grp * nblk);
+    r -= c * (grp * nblk);
+    first += c * grp;
+    ge = min((unsigned)grp, own - c * grp);
+  }
+  const unsigned j = r / ge;
+  bh = (int)(first + r - j * ge);
+  blk = (int)(heavy_last_index ? nblk - 1 - j : j);
 }
 
 // ------------------------------------------------------------------------------ forward
@@ -411,7 +430,7 @@ __global__ __launch_bounds__(256, D <= 64 && !FIRK ? 3 : 2) void flash_fwd_kerne
   const int N = p.N;
   const int nqb = (N + BM - 1) / BM;
   int bh, qblk;
-  map_block(nqb, p.B * p.H, CAUSAL, bh, qblk);
+  map_block(nqb, p.B * p.H, p.grp, CAUSAL, bh, qblk);
   const int b = bh / p.H, h = bh % p.H;
   const bf16* Q = static_cast<const bf16*>(p.q) + b * p.qsb + h * p.qsh;
   const bf16* K = static_cast<const bf16*>(p.k) + b * p.ksb + h * p.ksh;
@@ -919,7 +938,7 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dq_kernel(BwdParams p) {
   const int N = p.N;
   const int nqb = (N + BM - 1) / BM;
   int bh, qblk;
-  map_block(nqb, p.B * p.H, CAUSAL, bh, qblk);
+  map_block(nqb, p.B * p.H, p.grp, CAUSAL, bh, qblk);
   const int b = bh / p.H, h = bh % p.H;
   const bf16* Q = static_cast<const bf16*>(p.q) + b * p.qsb + h * p.qsh;
   const bf16* K = static_cast<const bf16*>(p.k) + b * p.ksb + h * p.ksh;
@@ -1348,7 +1367,7 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dkdv_kernel(BwdParams p) {
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave index, provably uniform
   const int N = p.N;
   int bh, kvb;
-  map_block(p.nkvb, p.B * p.H, false, bh, kvb);
+  map_block(p.nkvb, p.B * p.H, p.grp, false, bh, kvb);
   const int b = bh / p.H, h = bh % p.H;
   const bf16* K = static_cast<const bf16*>(p.k) + b * p.ksb + h * p.ksh;
   const bf16* V = static_cast<const bf16*>(p.v) + b * p.vsb + h * p.vsh;

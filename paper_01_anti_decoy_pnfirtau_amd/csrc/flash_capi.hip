@@ -116,6 +116,7 @@ extern "C" int pnfx_flash_fwd(const void* q, int64_t qsb, int64_t qsh, int64_t q
   FwdParams fp{q, k, v, o, o_lo, qsb, qsh, qsn, ksb, ksh, ksn, vsb, vsh, vsn, osb, osh, osn,
                M, Z, Nmax, tile_mask, static_cast<float*>(workspace), (int)B, (int)H, (int)N,
                (int)((N + 31) / 32), (int)((N + 63) / 64), tau, scale, gamma, has_gamma != 0};
+  fp.grp = slice_group(N, D);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   return dtype == PNFX_BF16 ? flash_fwd_bf16(fp, D, causal != 0, st)
                             : flash_fwd_f32(fp, D, causal != 0, has_gamma != 0, st);
@@ -144,7 +145,7 @@ extern "C" int pnfx_flash_fwd_fir(const void* q, int64_t qsb, int64_t qsh, int64
   FwdParams fp{q, k_raw, v, o, o_lo, qsb, qsh, qsn, ksb, ksh, ksn, vsb, vsh, vsn, osb, osh, osn,
                M, Z, nullptr, tile_mask, nullptr, (int)B, (int)H, (int)N,
                (int)((N + 31) / 32), (int)((N + 63) / 64), tau, scale, gamma, has_gamma != 0,
-               taps, (int)taps_rows, K};
+               taps, (int)taps_rows, K, slice_group(N, D)};
   return flash_fwd_fir_bf16(fp, D, causal != 0, reinterpret_cast<hipStream_t>(stream));
 }
 
@@ -200,7 +201,7 @@ extern "C" int pnfx_flash_bwd_stages(int stages, const void* q, int64_t qsb, int
                dqsb, dqsh, dqsn, dksb, dksh, dksn, dvsb, dvsh, dvsn,
                M, Z, tile_mask, rcbuf, parts, qs, ktact, amap, dtau,
                (int)B, (int)H, (int)N, (int)((N + 31) / 32), (int)((N + 63) / 64),
-               bwd_nkvb(N, D), tau, scale, gamma};
+               bwd_nkvb(N, D), tau, scale, gamma, slice_group(N, D)};
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   return dtype == PNFX_BF16 ? flash_bwd_bf16(bp, D, causal != 0, has_gamma != 0, stages, st)
                             : flash_bwd_f32(bp, D, causal != 0, has_gamma != 0, stages, st);
