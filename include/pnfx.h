@@ -185,8 +185,9 @@ int pnfx_flash_bwd(const void* q, int64_t qsb, int64_t qsh, int64_t qsn, const v
  * forms the per-row constants (and clears the key-tile activity bytes);
  * PNFX_BWD_DQ writes dq and the tau partials, stores each row's peak-tie share
  * and marks the 64-key tiles with an active tile_mask entry; PNFX_BWD_DKDV (which
- * reads all of these) writes dk, dv and (bf16) dtau.  For fp32 the DQ stage writes
- * dtau.  pnfx_flash_bwd is the mask PNFX_BWD_ALL.
+ * reads all of these) writes dk, dv and (bf16) dtau.  For fp32 the prepare stage has
+ * nothing to do and the DQ stage writes dtau (in a call with both, the DKDV stage's kernel
+ * does).  pnfx_flash_bwd is the mask PNFX_BWD_ALL.
  */
 #define PNFX_BWD_PREPARE 1
 #define PNFX_BWD_DKDV 2

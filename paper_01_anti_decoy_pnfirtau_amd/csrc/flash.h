@@ -71,7 +71,7 @@ inline int bwd_nkvb(int64_t N, int64_t D) {
   return (int)((N + bnk - 1) / bnk);
 }
 // Workspace of the backward: row constants, tau partials (fp64, one per wave of the bf16 dq
-// kernel, four per workgroup; the fp32 kernels use one per 64 rows), the peak-normalised
+// kernel, four per workgroup; the fp32 kernels use one per 32 rows), the peak-normalised
 // copy of Q that the bf16 dK/dV kernel reads, one activity byte per 64-key
 // tile, and the activity/tie map of the 32-query x 64-key sub-tiles (written by a dQ wave of
 // 32 rows, so only where the dQ kernel runs two 16-row blocks per wave: D <= 64).
@@ -99,7 +99,7 @@ int flash_fwd_bf16(const FwdParams& fp, int64_t D, bool causal, hipStream_t st);
 int flash_fwd_fir_bf16(const FwdParams& fp, int64_t D, bool causal, hipStream_t st);
 int flash_bwd_bf16(const BwdParams& bp, int64_t D, bool causal, bool has_gamma, int stages,
                    hipStream_t st);
-int flash_fwd_f32(const FwdParams& fp, int64_t D, bool causal, bool has_gamma, hipStream_t st);
+int flash_fwd_f32(const FwdParams& fp, int64_t D, bool causal, hipStream_t st);
 int flash_bwd_f32(const BwdParams& bp, int64_t D, bool causal, bool has_gamma, int stages,
                   hipStream_t st);
 

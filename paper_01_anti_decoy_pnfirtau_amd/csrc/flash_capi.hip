@@ -119,7 +119,7 @@ extern "C" int pnfx_flash_fwd(const void* q, int64_t qsb, int64_t qsh, int64_t q
   fp.grp = slice_group(N, D);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   return dtype == PNFX_BF16 ? flash_fwd_bf16(fp, D, causal != 0, st)
-                            : flash_fwd_f32(fp, D, causal != 0, has_gamma != 0, st);
+                            : flash_fwd_f32(fp, D, causal != 0, st);
 }
 
 extern "C" int pnfx_flash_fwd_fir(const void* q, int64_t qsb, int64_t qsh, int64_t qsn,

@@ -1,10 +1,12 @@
 """Work splits of the flash kernels at the sizes where they can go wrong: the dispatch order of
-(b, h) slices and query blocks."""
+(b, h) slices and query blocks, and the fp32 kernels' tiles, row alignment and last rows."""
+import numpy as np
 import pytest
 import torch
 
+from paper_01_anti_decoy_pnfirtau_amd import _lib, ops
 from paper_01_anti_decoy_pnfirtau_amd.hip_pnfirtau import flash_pn_fir_tau_attention
-from tests.helpers import seeded
+from tests.helpers import (F32_TOL, assert_close, assert_sum_close, flash_oracle, seeded, to_np64)
 
 pytestmark = pytest.mark.gpu
 
@@ -32,3 +34,70 @@ def test_flash_slices_do_not_depend_on_the_grid(dev, B, H, N, D):
         one = _grads(*(t[b:b + 1, h:h + 1] for t in (q, k, v)), 0.05, dO[b:b + 1, h:h + 1])
         for name, x, y in zip(("O", "dq", "dk", "dv"), whole, one):
             assert torch.equal(x[b, h], y[0, 0]), (name, b, h)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("aligned", [True, False])
+@pytest.mark.parametrize("D", [16, 32, 64, 128])
+@pytest.mark.parametrize("N", [1, 15, 17, 33, 64, 65, 129, 200])
+def test_flash_f32_edges_of_tiles_match_oracle(dev, N, D, aligned, causal):
+    """fp32 rows that end within a 16-row block, a 32-row workgroup or a 64-row tile, from
+    16-byte aligned rows and from rows that start at an odd float (staged by single floats)."""
+    print(f"[flash f32 N={N} D={D} aligned={aligned} causal={causal}]", flush=True)
+    B, H, tau, scale = 1, 2, 0.05, D ** -0.5
+    pad = 0 if aligned else 1
+    q, k, v, dO = (seeded((B, H, N, D + pad), 510 + i, torch.float32, dev)[..., pad:]
+                   for i in range(4))
+    o, dq, dk, dv, dt = _grads(q, k, v, tau, dO, causal)
+    Of, _, _, _, rdq, rdk, rdv, rdt, dabs = flash_oracle(q, k, v, tau, dO, scale, 0.5, causal)
+    for name, got, want in (("O", o, Of), ("dq", dq, rdq), ("dk", dk, rdk), ("dv", dv, rdv)):
+        assert_close(to_np64(got), want, F32_TOL, F32_TOL, name)
+    assert_sum_close(float(dt), rdt, dabs, F32_TOL, "dtau")
+
+
+def test_flash_f32_last_value_row_not_finite(dev):
+    """An infinite last row of V reaches the last query alone: the rows that pad the last tile do
+    not carry it to the others."""
+    N, D = 70, 64
+    q, k, v, _ = (seeded((1, 1, N, D), 520 + i, torch.float32, dev) for i in range(4))
+    k[..., -1, :] = q[..., -1, :]  # the last query attends to the last key
+    v[..., -1, :] = float("inf")
+    o = flash_pn_fir_tau_attention(q, k, v, torch.tensor(0.0, device=dev))
+    assert torch.isfinite(o[..., :64, :]).all()
+    assert not torch.isfinite(o[..., -1, :]).any()
+
+
+def test_flash_f32_backward_stages_called_separately(dev):
+    """The fp32 stages one by one: the dQ stage alone writes dtau, and the three together give
+    bitwise the outputs of one call."""
+    lib = _lib.lib()
+    B, H, N, D = 1, 3, 150, 64
+    q, k, v, dO = (seeded((B, H, N, D), 530 + i, torch.float32, dev) for i in range(4))
+    tau = torch.tensor(0.1, device=dev)
+    scale = float(1.0 / np.sqrt(D))
+    o, o_lo, M, Z, _, mask = torch.ops.pnfx.flash_fwd(q, k, v, tau, scale, 0.5, True, True, False,
+                                                      False)
+    nws = lib.pnfx_flash_bwd_workspace_size(B, H, N, D)
+
+    def run(stage_list):
+        ws = torch.empty(nws, device=dev, dtype=torch.uint8)
+        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+        dt = torch.zeros((), device=dev)
+        for st in stage_list:
+            rc = lib.pnfx_flash_bwd_stages(
+                st, *ops._ptr4(q), *ops._ptr4(k), *ops._ptr4(v), *ops._ptr4(o), None,
+                *ops._ptr4(dO), M.data_ptr(), Z.data_ptr(), mask.data_ptr(), *ops._ptr4(dq),
+                *ops._ptr4(dk), *ops._ptr4(dv), dt.data_ptr(), ws.data_ptr(), nws, B, H, N, D,
+                tau.data_ptr(), scale, 0.5, 1, 1, _lib.PNFX_F32,
+                torch.cuda.current_stream().cuda_stream)
+            assert rc == 0, lib.pnfx_last_error()
+        torch.cuda.synchronize()
+        return dq, dk, dv, dt
+
+    one = run([_lib.PNFX_BWD_ALL])
+    three = run([_lib.PNFX_BWD_PREPARE, _lib.PNFX_BWD_DQ, _lib.PNFX_BWD_DKDV])
+    for name, a, b in zip(("dq", "dk", "dv"), one, three):
+        assert torch.equal(a, b), name
+    assert float(three[3]) == pytest.approx(float(one[3]), rel=1e-6)  # another order of fp64 sums
+    dq_only = run([_lib.PNFX_BWD_PREPARE, _lib.PNFX_BWD_DQ])
+    assert torch.equal(dq_only[0], one[0]) and torch.equal(dq_only[3], three[3])
