@@ -180,6 +180,32 @@ int pnfx_flash_bwd(const void* q, int64_t qsb, int64_t qsh, int64_t qsn, const v
                    int dtype, void* stream);
 
 /*
+ * pnfx_flash_fwd and pnfx_flash_bwd for bf16 rows of any multiple of 8 up to 128 columns: those
+ * without a kernel of their own run the next larger one (16, 32, 64, 96 or 128 columns) over the
+ * D columns that exist, on the caller's tensors (no padded copies).  Same arguments and results; a
+ * forward and its backward go through the same pair.  The reference pads any D to a power of two
+ * by masked loads (src/triton_pnfirtau.py:839-841).
+ */
+int pnfx_flash_fwd_any(const void* q, int64_t qsb, int64_t qsh, int64_t qsn, const void* k,
+                   int64_t ksb, int64_t ksh, int64_t ksn, const void* v, int64_t vsb,
+                   int64_t vsh, int64_t vsn, void* o, int64_t osb, int64_t osh, int64_t osn,
+                   void* o_lo, float* M, float* Z, int32_t* Nmax, uint8_t* tile_mask,
+                   void* workspace, int64_t workspace_bytes, int64_t B, int64_t H,
+                   int64_t N, int64_t D, const float* tau, float scale, float gamma,
+                   int has_gamma, int causal, int dtype, void* stream);
+int pnfx_flash_bwd_any(const void* q, int64_t qsb, int64_t qsh, int64_t qsn, const void* k,
+                   int64_t ksb, int64_t ksh, int64_t ksn, const void* v, int64_t vsb,
+                   int64_t vsh, int64_t vsn, const void* o, int64_t osb, int64_t osh,
+                   int64_t osn, const void* o_lo, const void* dout, int64_t dosb, int64_t dosh, int64_t dosn,
+                   const float* M, const float* Z,
+                   const uint8_t* tile_mask, void* dq, int64_t dqsb, int64_t dqsh,
+                   int64_t dqsn, void* dk, int64_t dksb, int64_t dksh, int64_t dksn, void* dv,
+                   int64_t dvsb, int64_t dvsh, int64_t dvsn, float* dtau, void* workspace,
+                   int64_t workspace_bytes, int64_t B, int64_t H, int64_t N, int64_t D,
+                   const float* tau, float scale, float gamma, int has_gamma, int causal,
+                   int dtype, void* stream);
+
+/*
  * The three stages of pnfx_flash_bwd, callable separately (same arguments,
  * plus a stage mask), and run in this order on one workspace: PNFX_BWD_PREPARE
  * forms the per-row constants (and clears the key-tile activity bytes);

@@ -24,6 +24,7 @@ struct FwdParams {
   const float* fir_taps = nullptr;
   int fir_taps_rows = 0, fir_k = 0;
   int grp = 2;  // bf16: (b, h) slices per dispatch group (slice_group)
+  int d = 0;    // bf16: columns of a row of the operands (at most the kernel's head size)
 };
 
 struct BwdParams {
@@ -47,6 +48,7 @@ struct BwdParams {
   const float* tau;
   float scale, gamma;
   int grp = 2;  // bf16: (b, h) slices per dispatch group (slice_group)
+  int d = 0;    // bf16: columns of a row of the operands (at most the kernel's head size)
 };
 
 // (b, h) slices per dispatch group of the bf16 kernels: as many as keep the group's streamed pair of
@@ -58,6 +60,13 @@ struct BwdParams {
 inline int slice_group(int64_t N, int64_t D) {
   const int64_t g = (4ll << 20) / (N * D * 4);
   return (int)(g < 2 ? 2 : g > 64 ? 64 : g);
+}
+
+// Head size of the kernel that takes rows of D columns: D itself for the sizes with a kernel of their
+// own, the next of them, or 96, for others.
+constexpr bool own_kernel_dim(int64_t D) { return D == 16 || D == 32 || D == 64 || D == 128; }
+constexpr int kernel_dim(int64_t D) {
+  return D <= 16 ? 16 : D <= 32 ? 32 : D <= 64 ? 64 : D <= 96 ? 96 : 128;
 }
 
 // 16-row MFMA query blocks per wave of the bf16 dQ kernel (workgroups of four waves cover
@@ -80,7 +89,8 @@ inline int bwd_nkvb(int64_t N, int64_t D) {
 constexpr int64_t kAmapMaxN = 65536;
 struct BwdWorkspace {
   int64_t rc_bytes, parts_bytes, xt_bytes, kt_bytes, amap_bytes;
-  BwdWorkspace(int64_t B, int64_t H, int64_t N, int64_t D) {
+  BwdWorkspace(int64_t B, int64_t H, int64_t N, int64_t D_) {
+    const int64_t D = kernel_dim(D_);
     const int64_t rw = dq_rows_per_wg(D);
     const int64_t slots = B * H * ((N + rw - 1) / rw) * 4;
     rc_bytes = round256(B * H * N * 8 * 4);
@@ -96,6 +106,9 @@ struct BwdWorkspace {
 };
 
 int flash_fwd_bf16(const FwdParams& fp, int64_t D, bool causal, hipStream_t st);
+// Rows of fp.d columns, fp.d a multiple of 8 without a kernel of its own.
+int flash_fwd_ragged_bf16(const FwdParams& fp, bool causal, hipStream_t st);
+int flash_bwd_ragged_bf16(const BwdParams& bp, bool causal, bool has_gamma, hipStream_t st);
 int flash_fwd_fir_bf16(const FwdParams& fp, int64_t D, bool causal, hipStream_t st);
 int flash_bwd_bf16(const BwdParams& bp, int64_t D, bool causal, bool has_gamma, int stages,
                    hipStream_t st);

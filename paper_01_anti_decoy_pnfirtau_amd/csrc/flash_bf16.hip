@@ -120,6 +120,12 @@ __device__ __forceinline__ bf16x8 tr_frag(const bf16* tile, const FragLane& fl, 
   return __builtin_shufflevector(h[0], h[1], 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
+// Columns of an LDS tile row for head size D: at least the 32 of one MFMA k-step, and a power of two
+// for the swizzle (at D = 96 the last quarter of each row is neither filled nor read).
+constexpr int tile_cols(int D) { return D < 32 ? 32 : D == 96 ? 128 : D; }
+// k-steps of 32 columns of a product over the head dimension.
+constexpr int k_steps(int D) { return D < 32 ? 1 : D / 32; }
+
 // Direct global -> LDS staging of a 64-row tile (rows row0 .. row0 + 63 of an [N, D] bf16
 // slice with row stride sn) into the swizzled row-major layout, with global_load_lds_dwordx4:
 // no register staging and no LDS store instructions.  Each such load writes 16 bytes per
@@ -138,44 +144,48 @@ __device__ __forceinline__ void lds_dma16(const bf16* src, bf16* dst) {
 __device__ __forceinline__ int row_of_slot(int s) {  // inverse of slot_of
   return (s & 32) | ((s & 12) << 1) | ((s >> 2) & 4) | (s & 3);
 }
+// `d` <= D: the columns that the rows hold; chunks past them re-load the row's last one.
 template <int D, int DK>
 struct TileDma {
   static constexpr int CPR = DK / 8;      // 16-byte chunks per tile row
   static constexpr int NI = 64 * CPR / 256;  // loads per thread
+  static constexpr bool PART = D > 32 && D < DK;  // chunks past D are left alone
   int row[NI], col[NI];
   unsigned off[NI];  // byte offset of the lane's chunks from the tile's first row
-  __device__ __forceinline__ TileDma(int w, int lane, int64_t sn) {
+  __device__ __forceinline__ TileDma(int w, int lane, int64_t sn, int d = D) {
 #pragma unroll
     for (int j = 0; j < NI; ++j) {
       const int L = (4 * j + w) * 64 + lane;  // chunk index in the tile
       const int slot = L / CPR, pos = L % CPR;
       const int ch = pos ^ swz_rt<DK>(slot);
       row[j] = row_of_slot(slot);
-      col[j] = 8 * (ch % (D / 8));
+      col[j] = d == D ? 8 * (PART ? ch : ch % (D / 8)) : min(8 * ch, PART && ch >= D / 8 ? D : d - 8);
       off[j] = (unsigned)(2 * (row[j] * sn + col[j]));
     }
   }
   // A whole tile (row0 + 64 <= N) is a wave-uniform base plus 32-bit lane offsets, which the
   // load takes as scalar base + vector offset: no per-load address arithmetic.
   __device__ __forceinline__ void load(const bf16* src, int64_t sn, int row0, int N, bf16* tile,
-                                       int w) const {
+                                       int w, int d_last = D - 8) const {
     if (row0 + 64 <= N) {
       const char* base = reinterpret_cast<const char*>(src + (int64_t)row0 * sn);
 #pragma unroll
       for (int j = 0; j < NI; ++j)
-        lds_dma16(reinterpret_cast<const bf16*>(base + off[j]), tile + (4 * j + w) * 512);
+        if (!PART || col[j] < D)
+          lds_dma16(reinterpret_cast<const bf16*>(base + off[j]), tile + (4 * j + w) * 512);
     } else {
-      load_clamped(src, sn, row0, N, tile, w);
+      load_clamped(src, sn, row0, N, tile, w, d_last);
     }
   }
   // Any tile, from the row and column alone (fewer registers held across the loop, more
   // address arithmetic per load).
   __device__ __forceinline__ void load_clamped(const bf16* src, int64_t sn, int row0, int N,
-                                               bf16* tile, int w) const {
+                                               bf16* tile, int w, int d_last = D - 8) const {
 #pragma unroll
     for (int j = 0; j < NI; ++j) {
       const int r = min(row0 + row[j], N - 1);
-      lds_dma16(src + (int64_t)r * sn + col[j], tile + (4 * j + w) * 512);
+      if (!PART || col[j] < D)
+        lds_dma16(src + (int64_t)r * sn + min(col[j], d_last), tile + (4 * j + w) * 512);
     }
   }
 };
@@ -360,6 +370,7 @@ __global__ __launch_bounds__(256) void flash_key_norm_kernel(FwdParams p) {
                       (int64_t)(bh % p.H) * p.ksh + (int64_t)key * p.ksn;
 #pragma unroll
     for (int c = 0; c < D; c += 8) {
+      if (c >= p.d) continue;
       const u32x4 v = *reinterpret_cast<const u32x4*>(row + c);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -404,12 +415,14 @@ constexpr int kMaxListTiles = 1024;
 // FIRK (D <= 64): p.k holds the raw keys, and each key tile is filtered in LDS (the causal
 // FIR of pnfx_fir_fwd, fused into the key-tile load) before its scores; see
 // pnfx_flash_fwd_fir.
-template <int D, bool CAUSAL, bool PS, bool COUNT, bool FIRK = false>
+// RAG: p.d < D columns per row (a multiple of 8); the others count as zero.
+template <int D, bool CAUSAL, bool PS, bool COUNT, bool FIRK = false, bool RAG = false>
 __global__ __launch_bounds__(256, D <= 64 && !FIRK ? 3 : 2) void flash_fwd_kernel(FwdParams p) {
+  const int d = RAG ? p.d : D;
   constexpr int BM = 128, BN = 64;
   constexpr bool BOUND = D <= 64 && !FIRK;  // the silent-tile bound (see flash_key_norm_kernel)
-  constexpr int DK = D < 32 ? 32 : D;
-  constexpr int KS = DK / 32;
+  constexpr int DK = tile_cols(D);
+  constexpr int KS = k_steps(D);
   constexpr int DB = D / 16;
   static_assert(!FIRK || D <= 64, "the fused FIR is built for d <= 64");
   // Two K/V tile buffers as separate LDS objects (see the dK/dV kernel), filled straight
@@ -456,7 +469,7 @@ __global__ __launch_bounds__(256, D <= 64 && !FIRK ? 3 : 2) void flash_fwd_kerne
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const int col = 32 * ks + 8 * g;
-      qf[qb][ks] = (row < N && col < D) ? ld16(Q + (int64_t)row * p.qsn + col) : zero_bf16x8();
+      qf[qb][ks] = (row < N && col < d) ? ld16(Q + (int64_t)row * p.qsn + col) : zero_bf16x8();
       if (bound) gram = mfma16x16x32(qf[qb][ks], qf[qb][ks], gram);
       if (PS) qf[qb][ks] = scale_frag(qf[qb][ks], scale);
     }
@@ -550,7 +563,7 @@ __global__ __launch_bounds__(256, D <= 64 && !FIRK ? 3 : 2) void flash_fwd_kerne
 
   // Software pipeline: tile t+1 streams from HBM/L2 straight into one LDS buffer while tile
   // t is computed from the other; one barrier per tile.
-  const TileDma<D, DK> kdma(w, lane, p.ksn), vdma(w, lane, p.vsn);
+  const TileDma<D, DK> kdma(w, lane, p.ksn, d), vdma(w, lane, p.vsn, d);
   auto load_tile = [&](int n, const KVBuf& bb) {
     if constexpr (FIRK) {
       // raw rows n - 8 .. n + 63, KCPR chunks each (72 KCPR chunks, 64 per wave and load);
@@ -569,9 +582,9 @@ __global__ __launch_bounds__(256, D <= 64 && !FIRK ? 3 : 2) void flash_fwd_kerne
         }
       }
     } else {
-      kdma.load(K, p.ksn, n, N, bb.k, w);
+      kdma.load(K, p.ksn, n, N, bb.k, w, d - 8);
     }
-    vdma.load(V, p.vsn, n, N, bb.v, w);
+    vdma.load(V, p.vsn, n, N, bb.v, w, d - 8);
   };
   // FIRK: the filter taps of this head, h[u] = taps[K - 1 - u] (scalar registers)
   float fh[7] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -742,6 +755,7 @@ __global__ __launch_bounds__(256, D <= 64 && !FIRK ? 3 : 2) void flash_fwd_kerne
     if (qrow < N) {
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
+        if (RAG && 16 * db + 4 * g >= d) break;
         bf16x4 o4, r4;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -804,7 +818,7 @@ __global__ __launch_bounds__(256) void flash_bwd_pre_kernel(BwdParams p) {
       p.ktact[i] = 0;
   }
   float dot = 0.f;
-  if (row < total) {
+  if (row < total && 8 * part < p.d) {
     const int64_t bh = row / p.N, i = row % p.N;
     const int64_t b = bh / p.H, h = bh % p.H;
     const int64_t ooff = b * p.osb + h * p.osh + i * p.osn + 8 * part;
@@ -916,14 +930,15 @@ __device__ __forceinline__ bool peak_tie(const f32x4 (&s)[2][QB], const float (&
 // At D = 128 the dQ accumulators and the Q/dO fragments of 32 rows need more than the 256
 // registers a wave has at two workgroups per CU, so each wave takes 16 rows there (64-row
 // workgroups, two per CU) instead of running one 128-row workgroup per CU.
-template <int D, bool CAUSAL, bool PS>
+template <int D, bool CAUSAL, bool PS, bool RAG = false>
 __global__ __launch_bounds__(256, 2) void flash_bwd_dq_kernel(BwdParams p) {
+  const int d = RAG ? p.d : D;
   // Query rows per wave: 32 (two 16-row MFMA blocks) up to D = 64; 16 at D = 128, where the
   // dQ accumulators and the Q/dO fragments of 32 rows would not fit two workgroups per CU.
   constexpr int QB = dq_qblocks(D), RPW = 16 * QB;
   constexpr int BM = 4 * RPW, BN = 64;
-  constexpr int DK = D < 32 ? 32 : D;
-  constexpr int KS = DK / 32;
+  constexpr int DK = tile_cols(D);
+  constexpr int KS = k_steps(D);
   constexpr int DB = D / 16;
   // Two K/V tile buffers as separate LDS objects (see the dK/dV kernel), filled straight
   // from global memory.
@@ -986,10 +1001,10 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dq_kernel(BwdParams p) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const int col = 32 * ks + 8 * g;
-      const bool ok = rok && col < D;
+      const bool ok = rok && col < d;
       qf[qb][ks] = ok ? ld16(Q + (int64_t)row * p.qsn + col) : zero_bf16x8();
       dof[qb][ks] = ok ? ld16(dO + (int64_t)row * p.dosn + col) : zero_bf16x8();
-      if (ok)
+      if (rok && col < D)  // (zeros past d)
         *reinterpret_cast<bf16x8*>(Qs + (int64_t)row * D + col) =
             scale_frag(qf[qb][ks], __builtin_amdgcn_ldexpf(1.f, -rE[qb]));
       if (PS) qf[qb][ks] = scale_frag(qf[qb][ks], sc_e[qb]);  // a power of two: exact
@@ -1059,10 +1074,10 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dq_kernel(BwdParams p) {
     return ident ? e : __builtin_amdgcn_readfirstlane((int)tl_s[min(e, nlist - 1)]);
   };
 
-  const TileDma<D, DK> kdma(w, lane, p.ksn), vdma(w, lane, p.vsn);
+  const TileDma<D, DK> kdma(w, lane, p.ksn, d), vdma(w, lane, p.vsn, d);
   auto load_tile = [&](int n, const KVBuf& bb) {
-    kdma.load(K, p.ksn, n, N, bb.k, w);
-    vdma.load(V, p.vsn, n, N, bb.v, w);
+    kdma.load(K, p.ksn, n, N, bb.k, w, d - 8);
+    vdma.load(V, p.vsn, n, N, bb.v, w, d - 8);
   };
   // Entry e of the list: computed from buffer bc while the next tile streams into buffer bn.
   auto step = [&](int e, const KVBuf& bc, const KVBuf& bn) {
@@ -1192,6 +1207,7 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dq_kernel(BwdParams p) {
     if (qrow < N) {
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
+        if (RAG && 16 * db + 4 * g >= d) break;
         bf16x4 o4;
 #pragma unroll
         for (int i = 0; i < 4; ++i) o4[i] = (bf16)(acc[db][qb][i] * rowf);
@@ -1339,14 +1355,15 @@ __device__ __forceinline__ void dtau_sum(const double* partials, int64_t n, floa
   if (tid == 0) dtau[0] = (float)(-((red[0] + red[1]) + (red[2] + red[3])));
 }
 
-template <int D, bool CAUSAL, bool PS>
+template <int D, bool CAUSAL, bool PS, bool RAG = false>
 __global__ __launch_bounds__(256, 2) void flash_bwd_dkdv_kernel(BwdParams p) {
+  const int d = RAG ? p.d : D;
   // The scores are peak-normalised per row (from the dQ kernel's copy Q 2^-e, which also
   // serves the dK product) and the weights formed from u9s; the tiles are Q 2^-e and dO.
   constexpr int KPW = DkdvCfg<D>::KPW, KB = DkdvCfg<D>::KB, BNK = DkdvCfg<D>::BNK;
   constexpr int BMQ = 64;
-  constexpr int DK = D < 32 ? 32 : D;
-  constexpr int KS = DK / 32;
+  constexpr int DK = tile_cols(D);
+  constexpr int KS = k_steps(D);
   constexpr int DB = D / 16;
   // Two LDS buffers, as separate objects: the compiler then knows that the direct-to-LDS
   // loads filling one buffer do not write the other, and does not make the reads of the
@@ -1412,7 +1429,7 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dkdv_kernel(BwdParams p) {
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const int col = 32 * ks + 8 * g;
-      const bool ok = key < N && col < D;
+      const bool ok = key < N && col < d;
       kf[kb][ks] = ok ? ld16(K + (int64_t)key * p.ksn + col) : zero_bf16x8();
       vf[kb][ks] = ok ? ld16(V + (int64_t)key * p.vsn + col) : zero_bf16x8();
       if (PS) kf[kb][ks] = scale_frag(kf[kb][ks], scale);
@@ -1447,14 +1464,14 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dkdv_kernel(BwdParams p) {
   // scores are masked), including their row constants.  D <= 64: whole tiles take a scalar
   // base plus the lanes' fixed 32-bit offsets; D = 128, at the register limit, forms every
   // address from the row and column.
-  const TileDma<D, DK> tq(w, lane, D), tdo(w, lane, p.dosn);
+  const TileDma<D, DK> tq(w, lane, D), tdo(w, lane, p.dosn, d);
   auto load_tile = [&](int m, const QBuf& bb) {
     if (D <= 64) {
       tq.load(Qsc, D, m, N, bb.q, w);
-      tdo.load(dO, p.dosn, m, N, bb.o, w);
+      tdo.load(dO, p.dosn, m, N, bb.o, w, d - 8);
     } else {
       tq.load_clamped(Qsc, D, m, N, bb.q, w);
-      tq.load_clamped(dO, p.dosn, m, N, bb.o, w);
+      tq.load_clamped(dO, p.dosn, m, N, bb.o, w, d - 8);
     }
     const int row = min(m + lane, N - 1);
     lds_dma4(RCgw + row, bb.rc + w * BMQ);
@@ -1563,6 +1580,7 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dkdv_kernel(BwdParams p) {
     if (key < N) {
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
+        if (RAG && 16 * db + 4 * g >= d) break;
         bf16x4 k4, v4;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -1676,6 +1694,53 @@ int launch_bwd_d(const BwdParams& bp_in, bool causal, bool has_gamma, int stages
   return PNFX_OK;
 }
 
+// Rows of fewer columns than the kernel's head size: the same kernels with the range tests of RAG, no
+// scale folded in (PS) whatever it is, so that the backward recomputes the forward's scores.  The
+// tests lie in the prologue and epilogue; the loop is that of the full rows.  Padded copies of the
+// operands instead (and slices of the results) took 110 of 229 us at B=4 H=8 N=1000 d=80, where
+// this takes 103 us in all; 96 columns rather than 128 save a quarter of the products.
+template <int D>
+int launch_fwd_ragged(const FwdParams& fp, bool causal, hipStream_t st) {
+  if (fp.knorm && D <= 64 && fp.nk64 <= kMaxBoundTiles) {
+    const int64_t tiles = (int64_t)fp.B * fp.H * fp.nk64;
+    hipLaunchKernelGGL((flash_key_norm_kernel<D>), dim3((unsigned)((tiles + 3) / 4)), dim3(256), 0,
+                       st, fp);
+  }
+  const dim3 grid((unsigned)((fp.N + 127) / 128 * fp.B * fp.H)), block(256);
+  const bool count = fp.Nmax != nullptr;
+  if (causal) {
+    if (count) hipLaunchKernelGGL((flash_fwd_kernel<D, true, false, true, false, true>), grid, block, 0, st, fp);
+    else hipLaunchKernelGGL((flash_fwd_kernel<D, true, false, false, false, true>), grid, block, 0, st, fp);
+  } else {
+    if (count) hipLaunchKernelGGL((flash_fwd_kernel<D, false, false, true, false, true>), grid, block, 0, st, fp);
+    else hipLaunchKernelGGL((flash_fwd_kernel<D, false, false, false, false, true>), grid, block, 0, st, fp);
+  }
+  return launch_status("pnfx_flash_fwd_any");
+}
+
+template <int D>
+int launch_bwd_ragged(const BwdParams& bp_in, bool causal, bool has_gamma, hipStream_t st) {
+  const dim3 block(256);
+  BwdParams bp = bp_in;
+  if (dq_qblocks(D) < 2) bp.amap = nullptr;
+  constexpr int DP = tile_cols(D) < 64 ? D : tile_cols(D);  // the prepare kernel's lanes per row: a power of two
+  const int rpb = 256 / (DP / 8);
+  const dim3 gpre((unsigned)(((int64_t)bp.B * bp.H * bp.N + rpb - 1) / rpb));
+  if (has_gamma) hipLaunchKernelGGL((flash_bwd_pre_kernel<DP, true>), gpre, block, 0, st, bp);
+  else hipLaunchKernelGGL((flash_bwd_pre_kernel<DP, false>), gpre, block, 0, st, bp);
+  const int rw = (int)dq_rows_per_wg(D);
+  const dim3 gdq((unsigned)((bp.N + rw - 1) / rw * bp.B * bp.H));
+  const dim3 gkv((unsigned)(bp.nkvb * bp.B * bp.H));
+  if (causal) {
+    hipLaunchKernelGGL((flash_bwd_dq_kernel<D, true, false, true>), gdq, block, 0, st, bp);
+    hipLaunchKernelGGL((flash_bwd_dkdv_kernel<D, true, false, true>), gkv, block, 0, st, bp);
+  } else {
+    hipLaunchKernelGGL((flash_bwd_dq_kernel<D, false, false, true>), gdq, block, 0, st, bp);
+    hipLaunchKernelGGL((flash_bwd_dkdv_kernel<D, false, false, true>), gkv, block, 0, st, bp);
+  }
+  return launch_status("pnfx_flash_bwd_any");
+}
+
 }  // namespace
 
 
@@ -1711,6 +1776,26 @@ int flash_bwd_bf16(const BwdParams& bp, int64_t D, bool causal, bool has_gamma, 
   }
   set_error("flash: head dim %lld not in {16, 32, 64, 128}", (long long)D);
   return PNFX_EUNSUPPORTED;
+}
+
+int flash_fwd_ragged_bf16(const FwdParams& fp, bool causal, hipStream_t st) {
+  switch (kernel_dim(fp.d)) {
+    case 16: return launch_fwd_ragged<16>(fp, causal, st);
+    case 32: return launch_fwd_ragged<32>(fp, causal, st);
+    case 64: return launch_fwd_ragged<64>(fp, causal, st);
+    case 96: return launch_fwd_ragged<96>(fp, causal, st);
+    default: return launch_fwd_ragged<128>(fp, causal, st);
+  }
+}
+
+int flash_bwd_ragged_bf16(const BwdParams& bp, bool causal, bool has_gamma, hipStream_t st) {
+  switch (kernel_dim(bp.d)) {
+    case 16: return launch_bwd_ragged<16>(bp, causal, has_gamma, st);
+    case 32: return launch_bwd_ragged<32>(bp, causal, has_gamma, st);
+    case 64: return launch_bwd_ragged<64>(bp, causal, has_gamma, st);
+    case 96: return launch_bwd_ragged<96>(bp, causal, has_gamma, st);
+    default: return launch_bwd_ragged<128>(bp, causal, has_gamma, st);
+  }
 }
 
 }  // namespace pnfx

@@ -31,11 +31,14 @@ int check_operand(const char* name, const void* p, int64_t sb, int64_t sh, int64
   return PNFX_OK;
 }
 
-int check_shape(int64_t B, int64_t H, int64_t N, int64_t D) {
+int check_shape(int64_t B, int64_t H, int64_t N, int64_t D, bool any = false) {
   PNFX_REQUIRE(B >= 1 && H >= 1 && N >= 1, "flash: bad shape B=%lld H=%lld N=%lld", (long long)B,
                (long long)H, (long long)N);
-  PNFX_REQUIRE(D == 16 || D == 32 || D == 64 || D == 128, "flash: head dim %lld not in {16,32,64,128}",
-               (long long)D);
+  if (any)
+    PNFX_REQUIRE(D >= 8 && D <= 128 && D % 8 == 0,
+                 "flash: head dim %lld not a multiple of 8 up to 128", (long long)D);
+  else
+    PNFX_REQUIRE(own_kernel_dim(D), "flash: head dim %lld not in {16,32,64,128}", (long long)D);
   PNFX_REQUIRE(B * H <= (1ll << 30) && N <= (1ll << 28) && B * H * ((N + 127) / 128) < (1ll << 31),
                "flash: shape too large for the launch grid");
   return PNFX_OK;
@@ -90,7 +93,7 @@ extern "C" int64_t pnfx_flash_fwd_workspace_size(int64_t B, int64_t H, int64_t N
   return BwdWorkspace::round256(B * H * ((N + 63) / 64) * 4);
 }
 
-extern "C" int pnfx_flash_fwd(const void* q, int64_t qsb, int64_t qsh, int64_t qsn, const void* k,
+static int flash_fwd_impl(bool any, const void* q, int64_t qsb, int64_t qsh, int64_t qsn, const void* k,
                               int64_t ksb, int64_t ksh, int64_t ksn, const void* v, int64_t vsb,
                               int64_t vsh, int64_t vsn, void* o, int64_t osb, int64_t osh,
                               int64_t osn, void* o_lo, float* M, float* Z, int32_t* Nmax,
@@ -99,8 +102,8 @@ extern "C" int pnfx_flash_fwd(const void* q, int64_t qsb, int64_t qsh, int64_t q
                               float scale, float gamma, int has_gamma, int causal, int dtype,
                               void* stream) {
   int rc;
-  if ((rc = check_shape(B, H, N, D))) return rc;
-  PNFX_REQUIRE(dtype == PNFX_BF16 || dtype == PNFX_F32, "flash: unsupported dtype %d", dtype);
+  if ((rc = check_shape(B, H, N, D, any))) return rc;
+  PNFX_REQUIRE(dtype == PNFX_BF16 || (!any && dtype == PNFX_F32), "flash: unsupported dtype %d", dtype);
   if ((rc = check_operand("q", q, qsb, qsh, qsn, dtype))) return rc;
   if ((rc = check_operand("k", k, ksb, ksh, ksn, dtype))) return rc;
   if ((rc = check_operand("v", v, vsb, vsh, vsn, dtype))) return rc;
@@ -117,9 +120,36 @@ extern "C" int pnfx_flash_fwd(const void* q, int64_t qsb, int64_t qsh, int64_t q
                M, Z, Nmax, tile_mask, static_cast<float*>(workspace), (int)B, (int)H, (int)N,
                (int)((N + 31) / 32), (int)((N + 63) / 64), tau, scale, gamma, has_gamma != 0};
   fp.grp = slice_group(N, D);
+  fp.d = (int)D;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (!own_kernel_dim(D)) return flash_fwd_ragged_bf16(fp, causal != 0, st);
   return dtype == PNFX_BF16 ? flash_fwd_bf16(fp, D, causal != 0, st)
                             : flash_fwd_f32(fp, D, causal != 0, st);
+}
+
+extern "C" int pnfx_flash_fwd(const void* q, int64_t qsb, int64_t qsh, int64_t qsn, const void* k,
+                              int64_t ksb, int64_t ksh, int64_t ksn, const void* v, int64_t vsb,
+                              int64_t vsh, int64_t vsn, void* o, int64_t osb, int64_t osh, int64_t
+                              osn, void* o_lo, float* M, float* Z, int32_t* Nmax, uint8_t*
+                              tile_mask, void* workspace, int64_t workspace_bytes, int64_t B,
+                              int64_t H, int64_t N, int64_t D, const float* tau, float scale,
+                              float gamma, int has_gamma, int causal, int dtype, void* stream) {
+  return flash_fwd_impl(false, q, qsb, qsh, qsn, k, ksb, ksh, ksn, v, vsb, vsh, vsn, o, osb, osh,
+      osn, o_lo, M, Z, Nmax, tile_mask, workspace, workspace_bytes, B, H, N, D, tau, scale, gamma,
+      has_gamma, causal, dtype, stream);
+}
+
+extern "C" int pnfx_flash_fwd_any(const void* q, int64_t qsb, int64_t qsh, int64_t qsn, const
+                                  void* k, int64_t ksb, int64_t ksh, int64_t ksn, const void* v,
+                                  int64_t vsb, int64_t vsh, int64_t vsn, void* o, int64_t osb,
+                                  int64_t osh, int64_t osn, void* o_lo, float* M, float* Z,
+                                  int32_t* Nmax, uint8_t* tile_mask, void* workspace, int64_t
+                                  workspace_bytes, int64_t B, int64_t H, int64_t N, int64_t D,
+                                  const float* tau, float scale, float gamma, int has_gamma, int
+                                  causal, int dtype, void* stream) {
+  return flash_fwd_impl(true, q, qsb, qsh, qsn, k, ksb, ksh, ksn, v, vsb, vsh, vsn, o, osb, osh,
+      osn, o_lo, M, Z, Nmax, tile_mask, workspace, workspace_bytes, B, H, N, D, tau, scale, gamma,
+      has_gamma, causal, dtype, stream);
 }
 
 extern "C" int pnfx_flash_fwd_fir(const void* q, int64_t qsb, int64_t qsh, int64_t qsn,
@@ -145,7 +175,7 @@ extern "C" int pnfx_flash_fwd_fir(const void* q, int64_t qsb, int64_t qsh, int64
   FwdParams fp{q, k_raw, v, o, o_lo, qsb, qsh, qsn, ksb, ksh, ksn, vsb, vsh, vsn, osb, osh, osn,
                M, Z, nullptr, tile_mask, nullptr, (int)B, (int)H, (int)N,
                (int)((N + 31) / 32), (int)((N + 63) / 64), tau, scale, gamma, has_gamma != 0,
-               taps, (int)taps_rows, K, slice_group(N, D)};
+               taps, (int)taps_rows, K, slice_group(N, D), (int)D};
   return flash_fwd_fir_bf16(fp, D, causal != 0, reinterpret_cast<hipStream_t>(stream));
 }
 
@@ -153,7 +183,7 @@ extern "C" int64_t pnfx_flash_bwd_workspace_size(int64_t B, int64_t H, int64_t N
   return BwdWorkspace(B, H, N, D).total();
 }
 
-extern "C" int pnfx_flash_bwd_stages(int stages, const void* q, int64_t qsb, int64_t qsh, int64_t qsn, const void* k,
+static int flash_bwd_impl(bool any, int stages, const void* q, int64_t qsb, int64_t qsh, int64_t qsn, const void* k,
                               int64_t ksb, int64_t ksh, int64_t ksn, const void* v, int64_t vsb,
                               int64_t vsh, int64_t vsn, const void* o, int64_t osb, int64_t osh,
                               int64_t osn, const void* o_lo, const void* dout, int64_t dosb,
@@ -167,8 +197,8 @@ extern "C" int pnfx_flash_bwd_stages(int stages, const void* q, int64_t qsb, int
                               int has_gamma, int causal, int dtype, void* stream) {
   int rc;
   PNFX_REQUIRE(stages > 0 && (stages & ~PNFX_BWD_ALL) == 0, "flash_bwd: bad stage mask %d", stages);
-  if ((rc = check_shape(B, H, N, D))) return rc;
-  PNFX_REQUIRE(dtype == PNFX_BF16 || dtype == PNFX_F32, "flash: unsupported dtype %d", dtype);
+  if ((rc = check_shape(B, H, N, D, any))) return rc;
+  PNFX_REQUIRE(dtype == PNFX_BF16 || (!any && dtype == PNFX_F32), "flash: unsupported dtype %d", dtype);
   if ((rc = check_operand("q", q, qsb, qsh, qsn, dtype))) return rc;
   if ((rc = check_operand("k", k, ksb, ksh, ksn, dtype))) return rc;
   if ((rc = check_operand("v", v, vsb, vsh, vsn, dtype))) return rc;
@@ -201,10 +231,48 @@ extern "C" int pnfx_flash_bwd_stages(int stages, const void* q, int64_t qsb, int
                dqsb, dqsh, dqsn, dksb, dksh, dksn, dvsb, dvsh, dvsn,
                M, Z, tile_mask, rcbuf, parts, qs, ktact, amap, dtau,
                (int)B, (int)H, (int)N, (int)((N + 31) / 32), (int)((N + 63) / 64),
-               bwd_nkvb(N, D), tau, scale, gamma, slice_group(N, D)};
+               bwd_nkvb(N, D), tau, scale, gamma, slice_group(N, D), (int)D};
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (!own_kernel_dim(D)) return flash_bwd_ragged_bf16(bp, causal != 0, has_gamma != 0, st);
   return dtype == PNFX_BF16 ? flash_bwd_bf16(bp, D, causal != 0, has_gamma != 0, stages, st)
                             : flash_bwd_f32(bp, D, causal != 0, has_gamma != 0, stages, st);
+}
+
+extern "C" int pnfx_flash_bwd_stages(int stages, const void* q, int64_t qsb, int64_t qsh, int64_t
+                                     qsn, const void* k, int64_t ksb, int64_t ksh, int64_t ksn,
+                                     const void* v, int64_t vsb, int64_t vsh, int64_t vsn, const
+                                     void* o, int64_t osb, int64_t osh, int64_t osn, const void*
+                                     o_lo, const void* dout, int64_t dosb, int64_t dosh, int64_t
+                                     dosn, const float* M, const float* Z, const uint8_t*
+                                     tile_mask, void* dq, int64_t dqsb, int64_t dqsh, int64_t
+                                     dqsn, void* dk, int64_t dksb, int64_t dksh, int64_t dksn,
+                                     void* dv, int64_t dvsb, int64_t dvsh, int64_t dvsn, float*
+                                     dtau, void* workspace, int64_t workspace_bytes, int64_t B,
+                                     int64_t H, int64_t N, int64_t D, const float* tau, float
+                                     scale, float gamma, int has_gamma, int causal, int dtype,
+                                     void* stream) {
+  return flash_bwd_impl(false, stages, q, qsb, qsh, qsn, k, ksb, ksh, ksn, v, vsb, vsh, vsn, o,
+      osb, osh, osn, o_lo, dout, dosb, dosh, dosn, M, Z, tile_mask, dq, dqsb, dqsh, dqsn, dk,
+      dksb, dksh, dksn, dv, dvsb, dvsh, dvsn, dtau, workspace, workspace_bytes, B, H, N, D, tau,
+      scale, gamma, has_gamma, causal, dtype, stream);
+}
+
+extern "C" int pnfx_flash_bwd_any(const void* q, int64_t qsb, int64_t qsh, int64_t qsn, const
+                                  void* k, int64_t ksb, int64_t ksh, int64_t ksn, const void* v,
+                                  int64_t vsb, int64_t vsh, int64_t vsn, const void* o, int64_t
+                                  osb, int64_t osh, int64_t osn, const void* o_lo, const void*
+                                  dout, int64_t dosb, int64_t dosh, int64_t dosn, const float* M,
+                                  const float* Z, const uint8_t* tile_mask, void* dq, int64_t
+                                  dqsb, int64_t dqsh, int64_t dqsn, void* dk, int64_t dksb,
+                                  int64_t dksh, int64_t dksn, void* dv, int64_t dvsb, int64_t
+                                  dvsh, int64_t dvsn, float* dtau, void* workspace, int64_t
+                                  workspace_bytes, int64_t B, int64_t H, int64_t N, int64_t D,
+                                  const float* tau, float scale, float gamma, int has_gamma, int
+                                  causal, int dtype, void* stream) {
+  return flash_bwd_impl(true, PNFX_BWD_ALL, q, qsb, qsh, qsn, k, ksb, ksh, ksn, v, vsb, vsh, vsn,
+      o, osb, osh, osn, o_lo, dout, dosb, dosh, dosn, M, Z, tile_mask, dq, dqsb, dqsh, dqsn, dk,
+      dksb, dksh, dksn, dv, dvsb, dvsh, dvsn, dtau, workspace, workspace_bytes, B, H, N, D, tau,
+      scale, gamma, has_gamma, causal, dtype, stream);
 }
 
 extern "C" int pnfx_flash_bwd(const void* q, int64_t qsb, int64_t qsh, int64_t qsn, const void* k,

@@ -197,12 +197,18 @@ std::pair<Tensor, Tensor> new_o_pair(const Tensor& q, bool o_bnhd, bool with_lo)
 
 const void* ptr_or_null(const Tensor& t) { return t.numel() ? t.data_ptr() : nullptr; }
 
-// Head sizes with a kernel of their own; any other size up to 128 is zero-padded to the next
-// one (as the reference pads D to BLOCK_D = next_pow2(max(D, 16)) with masked loads,
-// src/triton_pnfirtau.py:839-841): zero columns add exact zeros to every dot product, so the
-// scores, O and the gradients' real columns are those of the unpadded problem.
-bool kernel_head_dim(int64_t D) { return D == 16 || D == 32 || D == 64 || D == 128; }
-int64_t padded_head_dim(int64_t D) { return D <= 16 ? 16 : D <= 32 ? 32 : D <= 64 ? 64 : 128; }
+// Head sizes the kernels take as they are: 16, 32, 64, 128 and, in bf16, any multiple of 8 below
+// (pnfx_flash_fwd_any).  Any other size up to 128 is zero-padded to the next one (as the reference
+// pads D to BLOCK_D = next_pow2(max(D, 16)) with masked loads, src/triton_pnfirtau.py:839-841): zero
+// columns add exact zeros to every dot product, so the scores, O and the gradients' real columns
+// are those of the unpadded problem.
+bool kernel_head_dim(int64_t D, bool bf16) {
+  return D == 16 || D == 32 || D == 64 || D == 128 || (bf16 && D >= 8 && D < 128 && D % 8 == 0);
+}
+int64_t padded_head_dim(int64_t D, bool bf16) {
+  if (bf16) return (D + 7) / 8 * 8;
+  return D <= 16 ? 16 : D <= 32 ? 32 : D <= 64 ? 64 : 128;
+}
 Tensor pad_d(const Tensor& t, int64_t Dp) {
   return t.numel() ? at::constant_pad_nd(t, {0, Dp - t.size(-1)}) : t;
 }
@@ -223,10 +229,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> flash_fwd_cuda(
   const int code = dtype_code(q_in, "flash");
   const bool bf = code == PNFX_BF16;
   TORCH_CHECK_VALUE(q_in.dim() == 4, "q must be [B,H,N,D], got ", q_in.sizes());
-  if (!kernel_head_dim(q_in.size(3))) {
+  if (!kernel_head_dim(q_in.size(3), bf)) {
     const int64_t D = q_in.size(3);
     check_head_dim(D);
-    const int64_t Dp = padded_head_dim(D);
+    const int64_t Dp = padded_head_dim(D, bf);
     auto [o, o_lo, M, Z, Nm, mask] = flash_fwd_cuda(pad_d(q_in, Dp), pad_d(k_in, Dp),
                                                     pad_d(v_in, Dp), tau, scale, gamma, has_gamma,
                                                     causal, false, with_nmax);
@@ -255,7 +261,8 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> flash_fwd_cuda(
   if (nws) ws = at::empty({nws}, q.options().dtype(at::kByte));
   const c10::DeviceGuard guard(q.device());
   const Tensor t32 = tau32(tau, q);
-  check_rc(pnfx_flash_fwd(q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), k.data_ptr(),
+  check_rc((bf ? pnfx_flash_fwd_any : pnfx_flash_fwd)(
+                          q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), k.data_ptr(),
                           k.stride(0), k.stride(1), k.stride(2), v.data_ptr(), v.stride(0),
                           v.stride(1), v.stride(2), o.data_ptr(), o.stride(0), o.stride(1),
                           o.stride(2), bf ? o_lo.data_ptr() : nullptr, M.data_ptr<float>(),
@@ -291,10 +298,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> flash_bwd_cuda(
   const int code = dtype_code(q_in, "flash");
   const bool bf = code == PNFX_BF16;
   TORCH_CHECK_VALUE(q_in.dim() == 4, "q must be [B,H,N,D], got ", q_in.sizes());
-  if (!kernel_head_dim(q_in.size(3))) {
+  if (!kernel_head_dim(q_in.size(3), bf)) {
     const int64_t D = q_in.size(3);
     check_head_dim(D);
-    const int64_t Dp = padded_head_dim(D);
+    const int64_t Dp = padded_head_dim(D, bf);
     auto [dq, dk, dv, dt] = flash_bwd_cuda(
         pad_d(q_in, Dp), pad_d(k_in, Dp), pad_d(v_in, Dp), tau, pad_d(o_in, Dp),
         o_lo.numel() == o_in.numel() ? pad_d(o_lo, Dp) : o_lo, pad_d(do_in, Dp), M, Z, mask,
@@ -324,7 +331,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> flash_bwd_cuda(
   const int64_t wsb = pnfx_flash_bwd_workspace_size(B, H, N, D);
   Tensor ws = at::empty({wsb}, q.options().dtype(at::kByte));
   const Tensor t32 = tau32(tau, q);
-  check_rc(pnfx_flash_bwd(
+  check_rc((bf ? pnfx_flash_bwd_any : pnfx_flash_bwd)(
                q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), k.data_ptr(), k.stride(0),
                k.stride(1), k.stride(2), v.data_ptr(), v.stride(0), v.stride(1), v.stride(2),
                o.data_ptr(), o.stride(0), o.stride(1), o.stride(2),

@@ -85,8 +85,8 @@ def hip_pn_fir_tau_scores(
     return w
 
 
-# Head sizes up to this have flash kernels (16, 32, 64, 128, the others zero-padded to the next
-# one inside the ops); larger heads take _materialised_attention.
+# Head sizes up to this have flash kernels (16, 32, 64, 128 and, in bf16, every multiple of 8; the
+# others zero-padded to the next one inside the ops); larger heads take _materialised_attention.
 FLASH_MAX_HEAD_DIM = 128
 
 
@@ -173,9 +173,9 @@ def flash_pn_fir_tau_attention(
 
     Returns O [B, H, N, d] (contiguous).  scale defaults to 1/sqrt(d).
     Backward is deterministic (no atomics) and returns grads for q, k_tilde, v and
-    score_tau (src/triton_pnfirtau.py:814-983).  Any head size: 16, 32, 64 and 128 have
-    kernels, other sizes up to 128 are zero-padded to the next of these, and larger heads
-    take the materialised-score path (_materialised_attention).
+    score_tau (src/triton_pnfirtau.py:814-983).  Any head size: 16, 32, 64 and 128 and (bf16)
+    multiples of 8 have kernels, other sizes up to 128 are zero-padded to the next of these, and
+    larger heads take the materialised-score path (_materialised_attention).
     """
     if scale is None:
         scale = 1.0 / math.sqrt(q.shape[-1])

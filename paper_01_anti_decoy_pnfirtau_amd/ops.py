@@ -144,7 +144,9 @@ def _grad_like(t: Tensor) -> Tensor:
 
 @torch.library.register_fake("pnfx::flash_bwd")
 def _(q, k, v, tau, o, o_lo, do, M, Z, mask, scale, gamma, has_gamma, causal):
-    if q.shape[-1] not in (16, 32, 64, 128):  # padded head sizes: contiguous slices
+    d = q.shape[-1]
+    if d not in (16, 32, 64, 128) and not (q.dtype == torch.bfloat16 and d < 128 and d % 8 == 0):
+        # padded head sizes: contiguous slices
         return (q.new_empty(q.shape), k.new_empty(k.shape), v.new_empty(v.shape),
                 q.new_empty(1, dtype=torch.float32))
     return _grad_like(q), _grad_like(k), _grad_like(v), q.new_empty(1, dtype=torch.float32)

@@ -101,3 +101,32 @@ def test_flash_f32_backward_stages_called_separately(dev):
     assert float(three[3]) == pytest.approx(float(one[3]), rel=1e-6)  # another order of fp64 sums
     dq_only = run([_lib.PNFX_BWD_PREPARE, _lib.PNFX_BWD_DQ])
     assert torch.equal(dq_only[0], one[0]) and torch.equal(dq_only[3], three[3])
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("d", [8, 20, 24, 40, 56, 72, 80, 96, 100, 104, 120])
+@pytest.mark.parametrize("N,causal", [(1, True), (65, True), (300, True), (130, False)])
+def test_flash_ragged_head_is_the_padded_head(dev, d, N, causal, packed):
+    """Head sizes that are multiples of 8 run on the caller's rows (others padded to one), bitwise as the rows
+    zero-padded to the next size with a kernel of its own: garbage in the tiles' unused columns
+    (neighbouring heads' data in a packed projection) reaches nothing."""
+    print(f"[flash ragged d={d} N={N} causal={causal} packed={packed}]", flush=True)
+    B, H, tau, scale = 2, 3, 0.05, 0.3  # (a scale that no kernel folds into its operands)
+    full = 16 if d < 16 else 32 if d < 32 else 64 if d < 64 else 128
+    rows = seeded((B, N, 3, H, d), 540, torch.bfloat16, dev)
+    q, k, v = (rows[:, :, i].transpose(1, 2) for i in range(3))
+    if not packed:
+        q, k, v = (t.contiguous() for t in (q, k, v))
+    dO = seeded((B, H, N, d), 541, torch.bfloat16, dev)
+
+    def run(*ts):
+        leaves = [t.detach().requires_grad_() for t in ts[:3]]
+        t0 = torch.tensor(tau, device=dev, requires_grad=True)
+        o = flash_pn_fir_tau_attention(*leaves, t0, scale=scale, causal_mask=causal)
+        return [o.detach(), *torch.autograd.grad(o, [*leaves, t0], ts[3])]
+
+    got = run(q, k, v, dO)
+    want = run(*(torch.nn.functional.pad(t, (0, full - d)) for t in (q, k, v, dO)))
+    for name, a, b in zip(("O", "dq", "dk", "dv"), got, want):
+        assert torch.equal(a, b[..., :d]), name
+    assert torch.equal(got[4], want[4])
