@@ -54,6 +54,8 @@ def _declare(lib: ctypes.CDLL) -> None:
             + [vp, i64, i64, i64] * 3
             + [vp, vp, i64, i64, i64, i64, i64, vp, f32, f32, i32, i32, i32, vp], i32),
     }
+    sig["pnfx_flash_fwd_any"] = sig["pnfx_flash_fwd"]
+    sig["pnfx_flash_bwd_any"] = sig["pnfx_flash_bwd"]
     sig["pnfx_flash_bwd_stages"] = ([i32] + sig["pnfx_flash_bwd"][0], i32)
     bwd = sig["pnfx_flash_bwd"][0]  # pnfx_flash_bwd without (workspace, workspace_bytes)
     sig["pnfx_flash_bwd_noalloc"] = (bwd[:37] + bwd[39:], i32)
@@ -92,5 +94,5 @@ def exported_symbols() -> list[str]:
         "pnfx_pn_rows_fwd", "pnfx_pn_rows_bwd", "pnfx_flash_fwd", "pnfx_flash_fwd_fir",
         "pnfx_flash_fwd_workspace_size",
         "pnfx_flash_bwd_workspace_size", "pnfx_flash_bwd", "pnfx_flash_bwd_stages",
-        "pnfx_flash_bwd_noalloc",
+        "pnfx_flash_bwd_noalloc", "pnfx_flash_fwd_any", "pnfx_flash_bwd_any",
     ]
