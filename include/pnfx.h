@@ -96,6 +96,16 @@ int pnfx_pn_rows_bwd(const void* dw, int64_t dw_rs, const void* raw, int64_t raw
                      void* stream);
 
 /*
+ * Sum of n floats (x 16-byte aligned) in fp64 and a fixed order, rounded once to out32[0] or left
+ * in out64[0] (one of them given): the tau gradient from pnfx_pn_rows_bwd's row partials, which the
+ * reference sums in fp64 too (src/triton_pnfirtau.py:784).  workspace:
+ * pnfx_sum_f64_workspace_size(n) bytes, 32-byte aligned (0 bytes, NULL, up to 131072 floats).
+ */
+int64_t pnfx_sum_f64_workspace_size(int64_t n);
+int pnfx_sum_f64(const float* x, int64_t n, void* workspace, int64_t workspace_bytes, float* out32,
+                 double* out64, void* stream);
+
+/*
  * Flash pn_fir_tau attention forward (p = 10, peak gate), O(N) memory.
  *   q, k, v, o : [B, H, N, D] with strides (s?b, s?h, s?n, 1), same dtype; bf16:
  *                16-byte aligned, strides multiples of 8, row strides s?n < 2^25

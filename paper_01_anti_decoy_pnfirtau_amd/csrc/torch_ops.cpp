@@ -150,6 +150,25 @@ std::tuple<Tensor, Tensor> pn_rows_bwd_cuda(const Tensor& dw, const Tensor& raw,
   return {d.view(raw.sizes()), dt};
 }
 
+// Sum of an fp32 tensor in fp64, one element: rounded to fp32, or kept (wide).
+Tensor sum_f64_cuda(const Tensor& x_in, bool wide) {
+  TORCH_CHECK_TYPE(x_in.scalar_type() == at::kFloat, "sum_f64: x is ", x_in.scalar_type());
+  Tensor x = x_in.contiguous();
+  if (reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 != 0) x = x.clone();
+  Tensor out = at::empty({1}, x.options().dtype(wide ? at::kDouble : at::kFloat));
+  const int64_t n = x.numel();
+  if (n == 0) return out.zero_();
+  const c10::DeviceGuard guard(x.device());
+  const int64_t wsb = pnfx_sum_f64_workspace_size(n);
+  Tensor ws;
+  if (wsb) ws = at::empty({wsb}, x.options().dtype(at::kByte));
+  check_rc(pnfx_sum_f64(x.data_ptr<float>(), n, wsb ? ws.data_ptr() : nullptr, wsb,
+                        wide ? nullptr : out.data_ptr<float>(),
+                        wide ? out.data_ptr<double>() : nullptr, stream_of(x)),
+           "pnfx_sum_f64");
+  return out;
+}
+
 // ------------------------------------------------------------------------------ flash
 // Past this sequence length the forward records no silence map (N^2/2048 bytes per (b, h));
 // the backward then recomputes every causal tile.  Kept equal to ops.MASK_MAX_N.
@@ -464,8 +483,11 @@ class RowsFn : public torch::autograd::Function<RowsFn> {
                             ctx->saved_data["has_gamma"].toBool(),
                             ctx->saved_data["causal"].toBool());
     // fp64 sum of the row partials, as src/triton_pnfirtau.py:784
+    static auto sum = op("pnfx::sum_f64").typed<Tensor(const Tensor&, bool)>();
     none[0] = d;
-    none[1] = dt.sum(at::kDouble).to(s[1].device(), s[1].scalar_type()).view_as(s[1]);
+    none[1] = sum.call(dt, s[1].scalar_type() != at::kFloat)
+                  .to(s[1].device(), s[1].scalar_type())
+                  .view_as(s[1]);
     return none;
   }
 };
@@ -548,6 +570,7 @@ TORCH_LIBRARY(pnfx, m) {
         "bool causal) -> (Tensor, Tensor, Tensor, Tensor)");
   m.def("pn_rows_bwd(Tensor dw, Tensor raw, Tensor tau, Tensor M, Tensor Z, Tensor Nmax, "
         "float scale, float p, float gamma, bool has_gamma, bool causal) -> (Tensor, Tensor)");
+  m.def("sum_f64(Tensor x, bool wide) -> Tensor");
   m.def("flash_fwd(Tensor q, Tensor k, Tensor v, Tensor tau, float scale, float gamma, "
         "bool has_gamma, bool causal, bool o_bnhd, bool with_nmax) -> "
         "(Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)");
@@ -564,6 +587,7 @@ TORCH_LIBRARY_IMPL(pnfx, CUDA, m) {
   m.impl("fir_bwd", fir_bwd_cuda);
   m.impl("pn_rows_fwd", pn_rows_fwd_cuda);
   m.impl("pn_rows_bwd", pn_rows_bwd_cuda);
+  m.impl("sum_f64", sum_f64_cuda);
   m.impl("flash_fwd", flash_fwd_cuda);
   m.impl("flash_bwd", flash_bwd_cuda);
   m.impl("flash_fwd_fir", flash_fwd_fir_cuda);

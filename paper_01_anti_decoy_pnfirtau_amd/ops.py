@@ -121,6 +121,11 @@ def _(dw, raw, tau, M, Z, Nmax, scale, p, gamma, has_gamma, causal):
             torch.empty(R, device=raw.device, dtype=torch.float32))
 
 
+@torch.library.register_fake("pnfx::sum_f64")
+def _(x, wide):
+    return torch.empty(1, device=x.device, dtype=torch.float64 if wide else torch.float32)
+
+
 @torch.library.register_fake("pnfx::flash_fwd")
 def _(q, k, v, tau, scale, gamma, has_gamma, causal, o_bnhd, with_nmax):
     _check_qkv(q, k, v)

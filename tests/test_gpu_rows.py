@@ -73,3 +73,62 @@ def test_rows_of_length_one_and_many_rows(dev):
         g = torch.where(m > 0, m / (m + 0.5), torch.zeros_like(m))
         ref = P / (P.sum(-1, keepdim=True) + 1e-12) * g
         torch.testing.assert_close(w.float(), ref, rtol=2e-2, atol=2e-3)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("p", [10.0, 2.0, 3.5])
+@pytest.mark.parametrize("N", [1, 7, 9, 255, 257, 511, 513, 1023, 1025, 2051])
+def test_rows_ends_of_chunks_match_oracle(dev, dtype, N, p):
+    """Rows that start at any element and end within a 16-byte chunk, one to five register chunks
+    long, forward and backward."""
+    print(f"[rows N={N} p={p} {dtype}]", flush=True)
+    from paper_01_anti_decoy_pnfirtau_amd.hip_pnfirtau import hip_pn_fir_tau_scores
+    raw = seeded((1, 1, N, N), 30, dtype, dev, scale=2.0).requires_grad_()
+    dW = seeded((1, 1, N, N), 31, dtype, dev)
+    tau = torch.tensor(0.1, device=dev, requires_grad=True)
+    w = hip_pn_fir_tau_scores(raw, tau, scale=0.5, p=p, gamma=0.5, causal_mask=True)
+    w.backward(dW)
+    rn = to_np64(raw)
+    W, M, Z, Nm = O.pn_rows_fwd(rn, 0.1, 0.5, p, 0.5, True)
+    d_raw, dtr = O.pn_rows_bwd(to_np64(dW), rn, 0.1, M, Z, Nm, 0.5, p, 0.5, True)
+    if dtype == torch.float32:
+        assert_close(to_np64(w), W, F32_TOL, F32_TOL, "W")
+        assert_close(to_np64(raw.grad), d_raw, F32_TOL, F32_TOL, "d_raw")
+    else:
+        assert_bf16_close(to_np64(w), W, "W")
+        assert_bf16_close(to_np64(raw.grad), d_raw, "d_raw")
+    tol = F32_TOL if dtype == torch.float32 else BF16_ATOL
+    assert abs(float(tau.grad) - dtr.sum()) <= tol * max(1.0, np.abs(dtr).sum())
+
+
+@pytest.mark.parametrize("p,size", [(10.0, 1e-6), (10.0, 1e-3), (10.0, 1e3), (2.0, 1e-12), (2.0, 1e12)])
+def test_rows_backward_over_the_range_of_peaks(dev, p, size):
+    """The backward's power-of-two unit: peaks whose powers are far from 1, or below fp32's range
+    (the largest scores here are 4.4 times `size`: at 1e3 their tenth powers end at 3e36, and 7e3
+    overflows fp32 in the forward)."""
+    from paper_01_anti_decoy_pnfirtau_amd.hip_pnfirtau import hip_pn_fir_tau_scores
+    N = 96
+    raw = (seeded((1, 1, N, N), 32, torch.float32, dev).abs() * size).requires_grad_()
+    dW = seeded((1, 1, N, N), 33, torch.float32, dev)
+    tau = torch.tensor(0.0, device=dev, requires_grad=True)
+    w = hip_pn_fir_tau_scores(raw, tau, scale=1.0, p=p, gamma=0.5, causal_mask=True)
+    w.backward(dW)
+    rn = to_np64(raw)
+    W, M, Z, Nm = O.pn_rows_fwd(rn, 0.0, 1.0, p, 0.5, True)
+    d_raw, _ = O.pn_rows_bwd(to_np64(dW), rn, 0.0, M, Z, Nm, 1.0, p, 0.5, True)
+    assert_close(to_np64(w), W, F32_TOL, F32_TOL, "W")
+    # nine roundings of u^9 and those of dW - D: 2e-5 of the largest entry
+    assert_close(to_np64(raw.grad), d_raw, 2 * F32_TOL, 2 * F32_TOL, "d_raw")
+
+
+@pytest.mark.parametrize("n", [1, 3, 5, 4096, 16385, 131072, 131073, 400001])
+def test_sum_f64_is_the_double_sum(dev, n):
+    """pnfx::sum_f64 (the tau gradient from the row partials): one and two launches, odd lengths,
+    and a view that does not start on 16 bytes; fp64 sums agree to their own rounding."""
+    x = seeded((n + 1,), 34, torch.float32, dev)
+    for t in (x[:n], x[1:]):
+        want = float(t.double().sum())
+        bound = 1e-14 * float(t.double().abs().sum())
+        assert abs(float(torch.ops.pnfx.sum_f64(t, True)) - want) <= bound
+        got = torch.ops.pnfx.sum_f64(t, False)
+        assert got.dtype == torch.float32 and abs(float(got) - want) <= 6e-8 * abs(want) + bound
