@@ -106,6 +106,19 @@ int pnfx_sum_f64(const float* x, int64_t n, void* workspace, int64_t workspace_b
                  double* out64, void* stream);
 
 /*
+ * Weight gradient of a bias-free linear layer: dw[M, N] = sum over K rows of dy[k, m] x[k, n], fp32
+ * sums in a fixed order.
+ *   dy, x : bf16 [K, M] and [K, N], row strides dy_rs >= M, x_rs >= N (multiples of 8, below 2^24)
+ *   dw    : [M, N] contiguous, dtype PNFX_F32 (the sums) or PNFX_BF16 (rounded once)
+ *   M, N multiples of 8 up to 65536; all pointers 16-byte aligned
+ *   workspace : pnfx_linear_wgrad_workspace_size(M, N, K, dtype) bytes (0: may be NULL)
+ */
+int64_t pnfx_linear_wgrad_workspace_size(int64_t M, int64_t N, int64_t K, int dtype);
+int pnfx_linear_wgrad(const void* dy, int64_t dy_rs, const void* x, int64_t x_rs, void* dw,
+                      int64_t M, int64_t N, int64_t K, int dtype, void* workspace,
+                      int64_t workspace_bytes, void* stream);
+
+/*
  * Flash pn_fir_tau attention forward (p = 10, peak gate), O(N) memory.
  *   q, k, v, o : [B, H, N, D] with strides (s?b, s?h, s?n, 1), same dtype; bf16:
  *                16-byte aligned, strides multiples of 8, row strides s?n < 2^25

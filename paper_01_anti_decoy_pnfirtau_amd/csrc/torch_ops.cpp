@@ -169,6 +169,44 @@ Tensor sum_f64_cuda(const Tensor& x_in, bool wide) {
   return out;
 }
 
+// ----------------------------------------------------------------------------- linear
+// dY^T X over bf16 rows [K, M] and [K, N]: fp32 (wide) or rounded to bf16.
+Tensor linear_wgrad_cuda(const Tensor& dy_in, const Tensor& x_in, bool wide) {
+  TORCH_CHECK_TYPE(dy_in.scalar_type() == at::kBFloat16 && x_in.scalar_type() == at::kBFloat16,
+                   "linear_wgrad: dy is ", dy_in.scalar_type(), ", x is ", x_in.scalar_type(),
+                   " (bfloat16)");
+  TORCH_CHECK_VALUE(dy_in.dim() == 2 && x_in.dim() == 2 && dy_in.size(0) == x_in.size(0) &&
+                        dy_in.device() == x_in.device(),
+                    "linear_wgrad: dy ", dy_in.sizes(), " and x ", x_in.sizes(),
+                    " must be [K, M] and [K, N] on one device");
+  const int64_t K = dy_in.size(0), M = dy_in.size(1), N = x_in.size(1);
+  const auto rows = [](const Tensor& t) {
+    const bool ok = t.stride(1) == 1 && t.stride(0) >= t.size(1) && t.stride(0) % 8 == 0 &&
+                    t.stride(0) < (1 << 24) && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+    return ok ? t : t.clone(at::MemoryFormat::Contiguous);
+  };
+  const Tensor dy = rows(dy_in), x = rows(x_in);
+  const auto f32 = dy.options().dtype(at::kFloat);
+  Tensor dw = at::empty({M, N}, wide ? f32 : dy.options());
+  if (K == 0 || M * N == 0) return dw.zero_();
+  const c10::DeviceGuard guard(dy.device());
+  const int code = wide ? PNFX_F32 : PNFX_BF16;
+  const int64_t wsb = pnfx_linear_wgrad_workspace_size(M, N, K, code);
+  Tensor ws;
+  if (wsb) ws = at::empty({wsb}, dy.options().dtype(at::kByte));
+  check_rc(pnfx_linear_wgrad(dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), dw.data_ptr(),
+                             M, N, K, code, wsb ? ws.data_ptr() : nullptr, wsb, stream_of(dy)),
+           "pnfx_linear_wgrad");
+  return dw;
+}
+
+// x W^T with bf16 x and W in bf16 or fp32 (rounded to bf16): the forward of LinearFn below.
+Tensor linear_cuda(const Tensor& x, const Tensor& w) {
+  TORCH_CHECK_TYPE(x.scalar_type() == at::kBFloat16, "linear: x is ", x.scalar_type(),
+                   " (bfloat16)");
+  return at::linear(x, w.to(at::kBFloat16));
+}
+
 // ------------------------------------------------------------------------------ flash
 // Past this sequence length the forward records no silence map (N^2/2048 bytes per (b, h));
 // the backward then recomputes every causal tile.  Kept equal to ops.MASK_MAX_N.
@@ -446,6 +484,47 @@ Tensor fir_fwd_autograd(const Tensor& x, const Tensor& taps) {
   return FirFn::apply(x, taps);
 }
 
+// x W^T for bf16 rows x and a bf16 or fp32 weight without bias, with the weight gradient from
+// pnfx_linear_wgrad in W's own type.
+class LinearFn : public torch::autograd::Function<LinearFn> {
+ public:
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    const Tensor wb = w.to(at::kBFloat16);
+    ctx->save_for_backward({x, wb});
+    ctx->saved_data["w"] = w;  // for a differentiable backward only
+    return linear_op().call(x, wb);
+  }
+  static const c10::TypedOperatorHandle<Tensor(const Tensor&, const Tensor&)>& linear_op() {
+    static auto h = op("pnfx::linear").typed<Tensor(const Tensor&, const Tensor&)>();
+    return h;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list gy) {
+    static auto wgrad =
+        op("pnfx::linear_wgrad").typed<Tensor(const Tensor&, const Tensor&, bool)>();
+    variable_list out(2);
+    if (!gy[0].defined()) return out;
+    const auto s = ctx->get_saved_variables();
+    const Tensor w = ctx->saved_data["w"].toTensor();
+    const bool again = at::GradMode::is_enabled();  // create_graph: products autograd can follow
+    const Tensor wb = again ? w.to(at::kBFloat16) : s[1];
+    const Tensor g2 = gy[0].reshape({-1, w.size(0)}), x2 = s[0].reshape({-1, w.size(1)});
+    if (ctx->needs_input_grad(0)) out[0] = at::mm(g2, wb).view(s[0].sizes());
+    if (ctx->needs_input_grad(1))
+      out[1] = again ? at::mm(g2.t(), x2).to(w.scalar_type())
+                     : wgrad.call(g2, x2, w.scalar_type() == at::kFloat);
+    return out;
+  }
+};
+
+Tensor linear_autograd(const Tensor& x, const Tensor& w) {
+  if (!records({&x, &w})) {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    return LinearFn::linear_op().call(x, w);
+  }
+  return LinearFn::apply(x, w);
+}
+
 const auto& rows_fwd_op() {
   static auto h = op("pnfx::pn_rows_fwd")
                       .typed<std::tuple<Tensor, Tensor, Tensor, Tensor>(
@@ -571,6 +650,8 @@ TORCH_LIBRARY(pnfx, m) {
   m.def("pn_rows_bwd(Tensor dw, Tensor raw, Tensor tau, Tensor M, Tensor Z, Tensor Nmax, "
         "float scale, float p, float gamma, bool has_gamma, bool causal) -> (Tensor, Tensor)");
   m.def("sum_f64(Tensor x, bool wide) -> Tensor");
+  m.def("linear(Tensor x, Tensor w) -> Tensor");
+  m.def("linear_wgrad(Tensor dy, Tensor x, bool wide) -> Tensor");
   m.def("flash_fwd(Tensor q, Tensor k, Tensor v, Tensor tau, float scale, float gamma, "
         "bool has_gamma, bool causal, bool o_bnhd, bool with_nmax) -> "
         "(Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)");
@@ -588,6 +669,8 @@ TORCH_LIBRARY_IMPL(pnfx, CUDA, m) {
   m.impl("pn_rows_fwd", pn_rows_fwd_cuda);
   m.impl("pn_rows_bwd", pn_rows_bwd_cuda);
   m.impl("sum_f64", sum_f64_cuda);
+  m.impl("linear", linear_cuda);
+  m.impl("linear_wgrad", linear_wgrad_cuda);
   m.impl("flash_fwd", flash_fwd_cuda);
   m.impl("flash_bwd", flash_bwd_cuda);
   m.impl("flash_fwd_fir", flash_fwd_fir_cuda);
@@ -596,5 +679,6 @@ TORCH_LIBRARY_IMPL(pnfx, CUDA, m) {
 TORCH_LIBRARY_IMPL(pnfx, Autograd, m) {
   m.impl("fir_fwd", fir_fwd_autograd);
   m.impl("pn_rows_fwd", pn_rows_fwd_autograd);
+  m.impl("linear", linear_autograd);
   m.impl("flash_fwd", flash_fwd_autograd);
 }

@@ -27,6 +27,7 @@ from __future__ import annotations
 import math
 
 import torch
+from torch.nn.modules import module as nn_module
 
 from . import ops  # noqa: F401  (registers the pnfx:: ops)
 from .pnfirtau_attention import causal_fir, power_norm_peak_gate
@@ -83,6 +84,44 @@ def hip_pn_fir_tau_scores(
                                             float(gamma) if has_gamma else 0.0, has_gamma,
                                             bool(causal_mask))
     return w
+
+
+def split_wgrad_applies(rows: int, out_features: int, in_features: int) -> bool:
+    """Whether pnfx::linear_wgrad is the faster weight gradient: many rows over a small weight, where
+    one workgroup per output tile leaves the chip idle.  Measured on MI355X (us, this kernel against
+    the library product and its cast to fp32): 768x256 over 16384 rows 29 / 93, over 2048 12 / 17,
+    over 512 9.8 / 10.0; 1536x512 over 8192 42 / 55, over 2048 24 / 19; 768x768 over 8192 36 / 51,
+    over 2048 22 / 18; 1024x1024 over 8192 34 / 56; 2304x768 over 16384 127 / 124; 3072x1024 over
+    65536 1272 / 492.  Columns in whole 16-byte chunks."""
+    mn = out_features * in_features
+    return out_features % 8 == 0 and in_features % 8 == 0 and mn <= 128 * rows and mn <= 1 << 20
+
+
+def project(lin: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """``lin(x)``; in bf16 training, where split_wgrad_applies, with the weight gradient from
+    pnfx::linear_wgrad (the library's product everywhere else, and for any module or tensor that is
+    not a plain bias-free nn.Linear without hooks on plain tensors)."""
+    if not (torch.is_grad_enabled() and type(lin) is torch.nn.Linear and lin.bias is None
+            and lin.weight.requires_grad and x.is_cuda and not torch.compiler.is_compiling()):
+        return lin(x)
+    w = lin.weight
+    if torch.is_autocast_enabled("cuda"):
+        bf16 = (torch.get_autocast_dtype("cuda") == torch.bfloat16
+                and w.dtype in (torch.float32, torch.bfloat16)
+                and x.dtype in (torch.float32, torch.bfloat16))
+    else:
+        bf16 = x.dtype == w.dtype == torch.bfloat16
+    hooks = (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks
+             or lin._backward_pre_hooks or "forward" in lin.__dict__
+             or nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks
+             or nn_module._global_backward_hooks or nn_module._global_backward_pre_hooks)
+    plain = (torch.Tensor, torch.nn.Parameter)
+    if (not bf16 or hooks or type(w) not in plain or type(x) not in plain or x.dim() < 2
+            or x.shape[-1] != w.shape[1] or w.device != x.device
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or not split_wgrad_applies(x.numel() // max(1, x.shape[-1]), *w.shape)):
+        return lin(x)
+    return torch.ops.pnfx.linear.default(x.to(torch.bfloat16), w)
 
 
 # Head sizes up to this have flash kernels (16, 32, 64, 128 and, in bf16, every multiple of 8; the

@@ -126,6 +126,16 @@ def _(x, wide):
     return torch.empty(1, device=x.device, dtype=torch.float64 if wide else torch.float32)
 
 
+@torch.library.register_fake("pnfx::linear")
+def _(x, w):
+    return x.new_empty((*x.shape[:-1], w.shape[0]))
+
+
+@torch.library.register_fake("pnfx::linear_wgrad")
+def _(dy, x, wide):
+    return dy.new_empty((dy.shape[1], x.shape[1]), dtype=torch.float32 if wide else dy.dtype)
+
+
 @torch.library.register_fake("pnfx::flash_fwd")
 def _(q, k, v, tau, scale, gamma, has_gamma, causal, o_bnhd, with_nmax):
     _check_qkv(q, k, v)

@@ -168,18 +168,18 @@ class PnFirTauTritonMHA(PnFirTauMHA):
     """
 
     def forward(self, x: torch.Tensor, return_weights: bool = False):
-        from .hip_pnfirtau import hip_causal_fir, hip_pn_fir_tau_scores
+        from .hip_pnfirtau import hip_causal_fir, hip_pn_fir_tau_scores, project
 
         cfg = self.cfg
         B, N, D = x.shape
-        q, k_raw, v = self.qkv(x).split(D, dim=-1)
+        q, k_raw, v = project(self.qkv, x).split(D, dim=-1)
         k = self._split_heads(hip_causal_fir(k_raw, self.fir_taps))
         q, v = self._split_heads(q), self._split_heads(v)
         raw = torch.matmul(q, k.transpose(-2, -1))
         w = hip_pn_fir_tau_scores(raw, self.score_tau, scale=1.0 / math.sqrt(self.head_dim),
                                   p=cfg.p, gamma=cfg.silence_gamma, causal_mask=cfg.causal_mask)
         w = self.drop(w)
-        out = self.out(torch.matmul(w, v).transpose(1, 2).reshape(B, N, D))
+        out = project(self.out, torch.matmul(w, v).transpose(1, 2).reshape(B, N, D))
         return (out, w) if return_weights else out
 
 
@@ -200,7 +200,7 @@ class PnFirTauFlashMHA(PnFirTauMHA):
 
         cfg = self.cfg
         B, N, D = x.shape
-        q, k_raw, v = self.qkv(x).split(D, dim=-1)
+        q, k_raw, v = hp.project(self.qkv, x).split(D, dim=-1)
         if hp.fused_fir_forward_applies(q, k_raw, self.fir_taps, self.head_dim):
             # inference: the key FIR inside the forward's key-tile load (one launch, same bits)
             o = hp.fused_fir_flash_forward(self._split_heads(q), self._split_heads(k_raw),
@@ -212,4 +212,4 @@ class PnFirTauFlashMHA(PnFirTauMHA):
         q, v = self._split_heads(q), self._split_heads(v)
         o = hp._flash_attention(q, k, v, self.score_tau, 1.0 / math.sqrt(self.head_dim),
                                 cfg.silence_gamma, cfg.causal_mask, o_bnhd=True)
-        return self.out(o.transpose(1, 2).reshape(B, N, D))
+        return hp.project(self.out, o.transpose(1, 2).reshape(B, N, D))

@@ -1,0 +1,89 @@
+"""The projections' weight gradient (pnfx::linear_wgrad) and the module path that uses it."""
+import pytest
+import torch
+
+from paper_01_anti_decoy_pnfirtau_amd import PnFirConfig, PnFirTauFlashMHA, hip_pnfirtau
+from tests.helpers import seeded
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("wide", [True, False])
+@pytest.mark.parametrize("M,N,K", [(8, 8, 1), (24, 16, 63), (128, 128, 64), (136, 120, 65),
+                                   (192, 64, 513), (768, 256, 777), (256, 264, 5001)])
+def test_linear_wgrad(dev, M, N, K, wide):
+    print(f"[linear_wgrad {M}x{N} over {K} wide={wide}]", flush=True)
+    rows = seeded((K, M + N + 8), 1, torch.bfloat16, dev)  # dy and x as column ranges of wider rows
+    dy, x = rows[:, :M], rows[:, M:M + N]
+    if M % 8 == 0 and K > 64:
+        dy = dy.contiguous()
+    got = torch.ops.pnfx.linear_wgrad.default(dy, x, wide)
+    again = torch.ops.pnfx.linear_wgrad.default(dy, x, wide)
+    assert got.dtype == (torch.float32 if wide else torch.bfloat16) and torch.equal(got, again)
+    d64, x64 = dy.double().cpu(), x.double().cpu()
+    ref, mass = d64.T @ x64, d64.abs().T @ x64.abs()
+    # fp32 sums of exact products: at most K + 2 roundings of 2^-24 of the absolute sum
+    err = (got.double().cpu() - ref).abs()
+    bound = (K + 2) * 2.0 ** -24 * mass + (0 if wide else 2.0 ** -8 * ref.abs())
+    assert bool((err <= bound).all()), float((err - bound).max())
+
+
+def test_linear_wgrad_not_finite_last_row(dev):
+    """The rows past K repeat the last one in LDS: its infinity counts once, zeros elsewhere."""
+    K = 70
+    dy, x = seeded((K, 16), 2, torch.bfloat16, dev), seeded((K, 24), 3, torch.bfloat16, dev).abs()
+    dy[-1, 3] = float("inf")
+    got = torch.ops.pnfx.linear_wgrad.default(dy, x, True).cpu()
+    ref = (dy.double().cpu().T @ x.double().cpu())
+    assert torch.equal(torch.isinf(got), torch.isinf(ref)) and not torch.isnan(got).any()
+
+
+def _grads(m, x, dy, autocast):
+    with torch.autocast("cuda", torch.bfloat16, enabled=autocast):
+        y = m(x)
+    return [y, *torch.autograd.grad(y, [x, *m.parameters()], dy)]
+
+
+@pytest.mark.parametrize("B,N,D,H", [(2, 512, 64, 4), (3, 333, 64, 4), (16, 256, 128, 4)])
+@pytest.mark.parametrize("autocast", [True, False])
+def test_module_gradients_match_the_library_product(dev, monkeypatch, B, N, D, H, autocast):
+    """Module outputs are the same bits with the library's product; only the weight gradients differ,
+    by the bf16 rounding that the library's product makes."""
+    print(f"[project B={B} N={N} D={D} autocast={autocast}]", flush=True)
+    torch.manual_seed(0)
+    m = PnFirTauFlashMHA(PnFirConfig(d_model=D, n_heads=H)).to(dev)
+    x = seeded((B, N, D), 4, torch.float32, dev)
+    if not autocast:
+        m, x = m.bfloat16(), x.bfloat16()
+    x.requires_grad_()
+    dy = seeded((B, N, D), 5, torch.bfloat16, dev)
+    assert hip_pnfirtau.split_wgrad_applies(B * N, 3 * D, D)
+    got = _grads(m, x, dy, autocast)
+    monkeypatch.setattr(hip_pnfirtau, "split_wgrad_applies", lambda *a: False)
+    ref = _grads(m, x, dy, autocast)
+    names = ["y", "x", *[n for n, _ in m.named_parameters()]]
+    for name, a, b in zip(names, got, ref):
+        assert a.dtype == b.dtype and a.shape == b.shape, name
+        if name.endswith("weight"):  # one or two roundings to bf16, 2^-9 each, of either
+            assert (a - b).float().norm() <= 2.0 ** -7 * b.float().norm(), name
+        else:
+            assert torch.equal(a, b), name
+
+
+def test_project_keeps_hooks_and_second_order(dev, monkeypatch):
+    lin = torch.nn.Linear(64, 64, bias=False, device=dev, dtype=torch.bfloat16)
+    x = seeded((4, 256, 64), 6, torch.bfloat16, dev).requires_grad_()
+
+    def second():
+        y = hip_pnfirtau.project(lin, x)
+        gx, gw = torch.autograd.grad((y * y).sum(), [x, lin.weight], create_graph=True)
+        return torch.autograd.grad(gx.square().sum() + gw.square().sum(), [x, lin.weight])
+
+    got = second()
+    calls = []
+    handle = lin.register_forward_hook(lambda *a: calls.append(1))
+    ref = second()  # a hooked module is called as it is
+    handle.remove()
+    assert calls == [1]
+    for a, b in zip(got, ref):
+        assert (a - b).float().norm() <= 2.0 ** -6 * b.float().norm()
