@@ -67,6 +67,10 @@ int pnfx_fir_fwd(const void* x, int64_t sb, int64_t sh, int64_t sn, void* y, int
 int pnfx_fir_bwd(const void* gy, int64_t sb, int64_t sh, int64_t sn, void* gx, int64_t B,
                  int64_t H, int64_t N, int64_t C, const float* taps, int64_t taps_rows, int K,
                  int dtype, void* stream);
+/* pnfx_fir_bwd into rows of any strides (a range of a wider tensor's columns, say). */
+int pnfx_fir_bwd_into(const void* gy, int64_t sb, int64_t sh, int64_t sn, void* gx, int64_t gxb,
+                      int64_t gxh, int64_t gxn, int64_t B, int64_t H, int64_t N, int64_t C,
+                      const float* taps, int64_t taps_rows, int K, int dtype, void* stream);
 
 /*
  * Row-fused rectified power-norm score -> weight, rows of a square [.., N, N]

@@ -56,6 +56,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     }
     sig["pnfx_sum_f64_workspace_size"] = ([i64], i64)
     sig["pnfx_sum_f64"] = ([vp, i64, vp, i64, vp, vp, vp], i32)
+    sig["pnfx_fir_bwd_into"] = ([vp, i64, i64, i64] * 2 + [i64, i64, i64, i64, vp, i64, i32, i32, vp],
+                                i32)
     sig["pnfx_linear_wgrad_workspace_size"] = ([i64, i64, i64, i32], i64)
     sig["pnfx_linear_wgrad"] = ([vp, i64, vp, i64, vp, i64, i64, i64, i32, vp, i64, vp], i32)
     sig["pnfx_flash_fwd_any"] = sig["pnfx_flash_fwd"]
@@ -100,5 +102,5 @@ def exported_symbols() -> list[str]:
         "pnfx_flash_bwd_workspace_size", "pnfx_flash_bwd", "pnfx_flash_bwd_stages",
         "pnfx_flash_bwd_noalloc", "pnfx_flash_fwd_any", "pnfx_flash_bwd_any",
         "pnfx_sum_f64_workspace_size", "pnfx_sum_f64",
-        "pnfx_linear_wgrad_workspace_size", "pnfx_linear_wgrad",
+        "pnfx_linear_wgrad_workspace_size", "pnfx_linear_wgrad", "pnfx_fir_bwd_into",
     ]

@@ -69,6 +69,7 @@ struct FirArgs {
   const void* x;
   int64_t sb, sh, sn;
   void* y;
+  int64_t ysb, ysh, ysn;
   int64_t B, H, N, C;
   const float* taps;
   int64_t taps_rows;
@@ -115,7 +116,8 @@ __global__ __launch_bounds__(256) void fir_vec_kernel(FirArgs a) {
       win[w] = u32x4{0u, 0u, 0u, 0u};
     }
   }
-  T* ys = reinterpret_cast<T*>(a.y) + ((int64_t)bh * N + n0) * a.C + ch * VEC;
+  T* ys = reinterpret_cast<T*>(a.y) + (int64_t)b * a.ysb + (int64_t)hh * a.ysh +
+          (int64_t)n0 * a.ysn + ch * VEC;
   // Window rows in the order of increasing lag (newest first for the forward, oldest first
   // for the adjoint): each row is widened to fp32 once and feeds every output of the run
   // that uses it, as that output's next term.  Output j (row n = n0 + j) sits at window
@@ -155,7 +157,7 @@ __global__ __launch_bounds__(256) void fir_vec_kernel(FirArgs a) {
   else chain(std::integral_constant<bool, true>{});
 #pragma unroll
   for (int j = 0; j < RUN; ++j)
-    if (n0 + j < N) store_chunk<T>(ys + (int64_t)j * a.C, acc[j]);
+    if (n0 + j < N) store_chunk<T>(ys + (int64_t)j * a.ysn, acc[j]);
 }
 
 // One thread per output element; any channel stride / alignment.
@@ -175,7 +177,7 @@ __global__ __launch_bounds__(256) void fir_scalar_kernel(FirArgs a, int64_t sc) 
     if (m < 0 || m >= a.N) break;
     acc = __builtin_fmaf(to_f32(xs[m * a.sn]), tp[a.K - 1 - u], acc);
   }
-  reinterpret_cast<T*>(a.y)[(bh * a.N + n) * a.C + c] = from_f32<T>(acc);
+  reinterpret_cast<T*>(a.y)[b * a.ysb + hh * a.ysh + n * a.ysn + c] = from_f32<T>(acc);
 }
 
 template <typename T, bool ADJ>
@@ -183,7 +185,8 @@ int launch_fir(const FirArgs& a, hipStream_t st) {
   constexpr int VEC = Chunk<T>::VEC;
   const bool vec_ok = (reinterpret_cast<uintptr_t>(a.x) % 16 == 0) &&
                       (reinterpret_cast<uintptr_t>(a.y) % 16 == 0) && a.C % VEC == 0 &&
-                      a.sb % VEC == 0 && a.sh % VEC == 0 && a.sn % VEC == 0;
+                      a.sb % VEC == 0 && a.sh % VEC == 0 && a.sn % VEC == 0 &&
+                      a.ysb % VEC == 0 && a.ysh % VEC == 0 && a.ysn % VEC == 0;
   const int64_t per_slice = ((a.N + RUN - 1) / RUN) * (a.C / VEC);
   if (vec_ok && per_slice < (1ll << 30) && a.B * a.H < 65536 && a.N < (1ll << 30)) {
     const dim3 grid((unsigned)((per_slice + 255) / 256), (unsigned)(a.B * a.H));
@@ -199,9 +202,9 @@ int launch_fir(const FirArgs& a, hipStream_t st) {
   return launch_status(ADJ ? "pnfx_fir_bwd" : "pnfx_fir_fwd");
 }
 
-int fir_entry(bool adj, const void* x, int64_t sb, int64_t sh, int64_t sn, void* y, int64_t B,
-              int64_t H, int64_t N, int64_t C, const float* taps, int64_t taps_rows, int K,
-              int dtype, void* stream) {
+int fir_entry(bool adj, const void* x, int64_t sb, int64_t sh, int64_t sn, void* y, int64_t ysb,
+              int64_t ysh, int64_t ysn, int64_t B, int64_t H, int64_t N, int64_t C,
+              const float* taps, int64_t taps_rows, int K, int dtype, void* stream) {
   PNFX_REQUIRE(x && y && taps, "fir: null pointer");
   PNFX_REQUIRE(B >= 0 && H >= 1 && N >= 0 && C >= 0, "fir: bad shape B=%lld H=%lld N=%lld C=%lld",
                (long long)B, (long long)H, (long long)N, (long long)C);
@@ -209,7 +212,7 @@ int fir_entry(bool adj, const void* x, int64_t sb, int64_t sh, int64_t sn, void*
   PNFX_REQUIRE(taps_rows == 1 || taps_rows == H, "fir: taps_rows=%lld must be 1 or H=%lld",
                (long long)taps_rows, (long long)H);
   if (B * H * N * C == 0) return PNFX_OK;
-  FirArgs a{x, sb, sh, sn, y, B, H, N, C, taps, taps_rows, K};
+  FirArgs a{x, sb, sh, sn, y, ysb, ysh, ysn, B, H, N, C, taps, taps_rows, K};
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (dtype == PNFX_BF16) return adj ? launch_fir<bf16, true>(a, st) : launch_fir<bf16, false>(a, st);
   if (dtype == PNFX_F32) return adj ? launch_fir<float, true>(a, st) : launch_fir<float, false>(a, st);
@@ -223,11 +226,21 @@ int fir_entry(bool adj, const void* x, int64_t sb, int64_t sh, int64_t sn, void*
 extern "C" int pnfx_fir_fwd(const void* x, int64_t sb, int64_t sh, int64_t sn, void* y, int64_t B,
                             int64_t H, int64_t N, int64_t C, const float* taps, int64_t taps_rows,
                             int K, int dtype, void* stream) {
-  return pnfx::fir_entry(false, x, sb, sh, sn, y, B, H, N, C, taps, taps_rows, K, dtype, stream);
+  return pnfx::fir_entry(false, x, sb, sh, sn, y, H * N * C, N * C, C, B, H, N, C, taps, taps_rows, K, dtype, stream);
 }
 
 extern "C" int pnfx_fir_bwd(const void* gy, int64_t sb, int64_t sh, int64_t sn, void* gx,
                             int64_t B, int64_t H, int64_t N, int64_t C, const float* taps,
                             int64_t taps_rows, int K, int dtype, void* stream) {
-  return pnfx::fir_entry(true, gy, sb, sh, sn, gx, B, H, N, C, taps, taps_rows, K, dtype, stream);
+  return pnfx::fir_entry(true, gy, sb, sh, sn, gx, H * N * C, N * C, C, B, H, N, C, taps, taps_rows, K, dtype, stream);
+}
+
+extern "C" int pnfx_fir_bwd_into(const void* gy, int64_t sb, int64_t sh, int64_t sn, void* gx,
+                                 int64_t gxb, int64_t gxh, int64_t gxn, int64_t B, int64_t H,
+                                 int64_t N, int64_t C, const float* taps, int64_t taps_rows, int K,
+                                 int dtype, void* stream) {
+  PNFX_REQUIRE(gxn >= C, "fir: output rows of %lld elements at a stride of %lld", (long long)C,
+               (long long)gxn);
+  return pnfx::fir_entry(true, gy, sb, sh, sn, gx, gxb, gxh, gxn, B, H, N, C, taps, taps_rows, K,
+                         dtype, stream);
 }

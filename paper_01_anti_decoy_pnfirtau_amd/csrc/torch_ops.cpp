@@ -344,10 +344,13 @@ Tensor grad_like(const Tensor& t) {
   return at::empty({B, H, N, D}, t.options());
 }
 
-std::tuple<Tensor, Tensor, Tensor, Tensor> flash_bwd_cuda(
+// `into`: dQ, dK and dV, [B,H,N,D] views to write (head sizes with kernels of their own only), or
+// undefined.
+std::tuple<Tensor, Tensor, Tensor, Tensor> flash_bwd_into(
     const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, const Tensor& tau,
     const Tensor& o_in, const Tensor& o_lo, const Tensor& do_in, const Tensor& M, const Tensor& Z,
-    const Tensor& mask, double scale, double gamma, bool has_gamma, bool causal) {
+    const Tensor& mask, double scale, double gamma, bool has_gamma, bool causal,
+    std::array<Tensor, 3> into) {
   check_qkv(q_in, k_in, v_in);
   TORCH_CHECK_VALUE(o_in.sizes() == q_in.sizes() && do_in.sizes() == q_in.sizes(),
                     "flash_bwd: o ", o_in.sizes(), " / dO ", do_in.sizes(), " must match q ",
@@ -359,10 +362,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> flash_bwd_cuda(
     const int64_t D = q_in.size(3);
     check_head_dim(D);
     const int64_t Dp = padded_head_dim(D, bf);
-    auto [dq, dk, dv, dt] = flash_bwd_cuda(
+    auto [dq, dk, dv, dt] = flash_bwd_into(
         pad_d(q_in, Dp), pad_d(k_in, Dp), pad_d(v_in, Dp), tau, pad_d(o_in, Dp),
         o_lo.numel() == o_in.numel() ? pad_d(o_lo, Dp) : o_lo, pad_d(do_in, Dp), M, Z, mask,
-        scale, gamma, has_gamma, causal);
+        scale, gamma, has_gamma, causal, {});
     return {dq.narrow(3, 0, D).contiguous(), dk.narrow(3, 0, D).contiguous(),
             dv.narrow(3, 0, D).contiguous(), dt};
   }
@@ -374,14 +377,17 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> flash_bwd_cuda(
                            "dO", bf);
   const int64_t B = q.size(0), H = q.size(1), N = q.size(2), D = q.size(3);
   check_saved(M, "flash_bwd", "M", B * H * N, at::kFloat, q);
-  // Each gradient in its input's dimension order (see grad_like).
   check_saved(Z, "flash_bwd", "Z", B * H * N, at::kFloat, q);
   if (mask.numel()) {  // the forward's tile mask, or none (every causal tile recomputed)
     const auto ms = mask_shape(B, H, N);
     check_saved(mask, "flash_bwd", "mask", ms[0] * ms[1] * ms[2], at::kByte, q);
   }
-  // dQ, dK, dV and dtau, each its own allocation (returned to autograd as the inputs' grads)
-  Tensor dq = grad_like(q_in), dk = grad_like(k_in), dv = grad_like(v_in);
+  // Each gradient its own allocation (returned to autograd as the inputs' grads) in its input's
+  // dimension order (see grad_like), unless the caller has a place for it.
+  const auto out = [](const Tensor& given, const Tensor& like) {
+    return given.defined() ? given : grad_like(like);
+  };
+  Tensor dq = out(into[0], q_in), dk = out(into[1], k_in), dv = out(into[2], v_in);
   Tensor dtau = at::empty({1}, q.options().dtype(at::kFloat));
   if (B * H * N == 0) return {dq, dk, dv, dtau.zero_()};  // -(sum over no scores) = 0
   const c10::DeviceGuard guard(q.device());
@@ -401,6 +407,68 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> flash_bwd_cuda(
                (float)scale, (float)gamma, has_gamma, causal, code, stream_of(q)),
            "pnfx_flash_bwd");
   return {dq, dk, dv, dtau};
+}
+
+std::tuple<Tensor, Tensor, Tensor, Tensor> flash_bwd_cuda(
+    const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& tau, const Tensor& o,
+    const Tensor& o_lo, const Tensor& dout, const Tensor& M, const Tensor& Z, const Tensor& mask,
+    double scale, double gamma, bool has_gamma, bool causal) {
+  return flash_bwd_into(q, k, v, tau, o, o_lo, dout, M, Z, mask, scale, gamma, has_gamma, causal,
+                        {});
+}
+
+// Attention over projection rows qkv [B, N, 3 H d] (q, raw k, v; each its heads side by side): the
+// key FIR, then flash, as one pass of autograd.  Its backward writes dq and dv, and the FIR's
+// adjoint of dk, into their columns of one [B, N, 3 H d] gradient.
+Tensor rows_as_heads(const Tensor& rows, int64_t H) {  // [B, N, H d] -> [B, H, N, d]
+  return rows.view({rows.size(0), rows.size(1), H, rows.size(2) / H}).transpose(1, 2);
+}
+
+void check_qkv_rows(const Tensor& qkv, const Tensor& taps, int64_t H) {
+  TORCH_CHECK_TYPE(qkv.scalar_type() == at::kBFloat16, "attn_rows: qkv is ", qkv.scalar_type(),
+                   " (bfloat16)");
+  TORCH_CHECK_VALUE(qkv.dim() == 3 && qkv.is_contiguous() && qkv.numel() > 0 && H >= 1 &&
+                        qkv.size(2) % (3 * H) == 0,
+                    "attn_rows: qkv ", qkv.sizes(), " must be contiguous [B, N, 3 * ", H, " * d]");
+  TORCH_CHECK_VALUE(kernel_head_dim(qkv.size(2) / (3 * H), true) && taps.dim() == 1,
+                    "attn_rows: head dim ", qkv.size(2) / (3 * H), ", taps ", taps.sizes());
+}
+
+// o rows [B, N, H d], o_lo [B, H, N, d] over such rows, the filtered key rows, M, Z, tile mask
+std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> attn_rows_cuda(
+    const Tensor& qkv, const Tensor& taps, const Tensor& tau, int64_t H, double scale,
+    double gamma, bool has_gamma, bool causal) {
+  check_qkv_rows(qkv, taps, H);
+  const int64_t C = qkv.size(2) / 3;
+  const Tensor kf = fir_call(qkv.narrow(2, C, C), taps, false);
+  auto [o, o_lo, M, Z, Nm, mask] = flash_fwd_cuda(
+      rows_as_heads(qkv.narrow(2, 0, C), H), rows_as_heads(kf, H),
+      rows_as_heads(qkv.narrow(2, 2 * C, C), H), tau, scale, gamma, has_gamma, causal, true, false);
+  return {o.transpose(1, 2).view({qkv.size(0), qkv.size(1), C}), o_lo, kf, M, Z, mask};
+}
+
+std::tuple<Tensor, Tensor> attn_rows_bwd_cuda(
+    const Tensor& qkv, const Tensor& kf, const Tensor& taps, const Tensor& tau, const Tensor& o,
+    const Tensor& o_lo, const Tensor& dout, const Tensor& M, const Tensor& Z, const Tensor& mask,
+    double scale, double gamma, bool has_gamma, bool causal) {
+  const int64_t H = M.size(1), C = qkv.size(2) / 3;
+  check_qkv_rows(qkv, taps, H);
+  TORCH_CHECK_VALUE(dout.sizes() == o.sizes(), "attn_rows_bwd: dO has shape ", dout.sizes(),
+                    ", O ", o.sizes());
+  const c10::DeviceGuard guard(qkv.device());
+  Tensor d = at::empty(qkv.sizes(), qkv.options());
+  const Tensor dk_raw = d.narrow(2, C, C);
+  const auto heads = [&](int64_t i) { return rows_as_heads(qkv.narrow(2, i * C, C), H); };
+  auto [dq, dk, dv, dtau] = flash_bwd_into(
+      heads(0), rows_as_heads(kf, H), heads(2), tau, rows_as_heads(o, H), o_lo,
+      rows_as_heads(dout.contiguous(), H), M, Z, mask, scale, gamma, has_gamma, causal,
+      {rows_as_heads(d.narrow(2, 0, C), H), Tensor(), rows_as_heads(d.narrow(2, 2 * C, C), H)});
+  const Tensor t = taps.to(qkv.device(), at::kFloat).contiguous();
+  check_rc(pnfx_fir_bwd_into(dk.data_ptr(), dk.stride(0), 0, dk.stride(2), dk_raw.data_ptr(),
+                             dk_raw.stride(0), 0, dk_raw.stride(1), qkv.size(0), 1, qkv.size(1), C,
+                             t.data_ptr<float>(), 1, (int)t.size(0), PNFX_BF16, stream_of(qkv)),
+           "pnfx_fir_bwd_into");
+  return {d, dtau};
 }
 
 std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> flash_fwd_fir_cuda(
@@ -640,6 +708,62 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> flash_fwd_autograd(
   return {r[0], r[1], r[2], r[3], r[4], r[5]};
 }
 
+const auto& attn_rows_op() {
+  static auto h = op("pnfx::attn_rows")
+                      .typed<std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor>(
+                          const Tensor&, const Tensor&, const Tensor&, int64_t, double, double,
+                          bool, bool)>();
+  return h;
+}
+
+class AttnRowsFn : public torch::autograd::Function<AttnRowsFn> {
+ public:
+  static variable_list forward(AutogradContext* ctx, const Tensor& qkv, const Tensor& taps,
+                               const Tensor& tau, int64_t H, double scale, double gamma,
+                               bool has_gamma, bool causal) {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    auto [o, o_lo, kf, M, Z, mask] =
+        attn_rows_op().call(qkv, taps, tau, H, scale, gamma, has_gamma, causal);
+    ctx->mark_non_differentiable({o_lo, kf, M, Z, mask});
+    ctx->set_materialize_grads(false);
+    ctx->save_for_backward({qkv, kf, taps, tau, o, o_lo, M, Z, mask});
+    ctx->saved_data["scale"] = scale;
+    ctx->saved_data["gamma"] = gamma;
+    ctx->saved_data["has_gamma"] = has_gamma;
+    ctx->saved_data["causal"] = causal;
+    return {o, o_lo, kf, M, Z, mask};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list g) {
+    static auto bwd = op("pnfx::attn_rows_bwd")
+                          .typed<std::tuple<Tensor, Tensor>(
+                              const Tensor&, const Tensor&, const Tensor&, const Tensor&,
+                              const Tensor&, const Tensor&, const Tensor&, const Tensor&,
+                              const Tensor&, const Tensor&, double, double, bool, bool)>();
+    variable_list grads(8);
+    if (!g[0].defined()) return grads;
+    const auto s = ctx->get_saved_variables();
+    auto [d, dt] = bwd.call(s[0], s[1], s[2], s[3], s[4], s[5], g[0], s[6], s[7], s[8],
+                            ctx->saved_data["scale"].toDouble(),
+                            ctx->saved_data["gamma"].toDouble(),
+                            ctx->saved_data["has_gamma"].toBool(),
+                            ctx->saved_data["causal"].toBool());
+    grads[0] = d;
+    grads[2] = dt.to(s[3].device(), s[3].scalar_type()).view_as(s[3]);
+    return grads;
+  }
+};
+
+std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> attn_rows_autograd(
+    const Tensor& qkv, const Tensor& taps, const Tensor& tau, int64_t H, double scale,
+    double gamma, bool has_gamma, bool causal) {
+  if (!records({&qkv, &taps, &tau})) {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    return attn_rows_op().call(qkv, taps, tau, H, scale, gamma, has_gamma, causal);
+  }
+  auto r = AttnRowsFn::apply(qkv, taps, tau, H, scale, gamma, has_gamma, causal);
+  return {r[0], r[1], r[2], r[3], r[4], r[5]};
+}
+
 }  // namespace
 
 TORCH_LIBRARY(pnfx, m) {
@@ -658,6 +782,11 @@ TORCH_LIBRARY(pnfx, m) {
   m.def("flash_bwd(Tensor q, Tensor k, Tensor v, Tensor tau, Tensor o, Tensor o_lo, Tensor do, "
         "Tensor M, Tensor Z, Tensor mask, float scale, float gamma, bool has_gamma, bool causal) "
         "-> (Tensor, Tensor, Tensor, Tensor)");
+  m.def("attn_rows(Tensor qkv, Tensor taps, Tensor tau, int heads, float scale, float gamma, "
+        "bool has_gamma, bool causal) -> (Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)");
+  m.def("attn_rows_bwd(Tensor qkv, Tensor k, Tensor taps, Tensor tau, Tensor o, Tensor o_lo, "
+        "Tensor do, Tensor M, Tensor Z, Tensor mask, float scale, float gamma, bool has_gamma, "
+        "bool causal) -> (Tensor, Tensor)");
   m.def("flash_fwd_fir(Tensor q, Tensor k_raw, Tensor v, Tensor tau, Tensor taps, float scale, "
         "float gamma, bool has_gamma, bool causal, bool o_bnhd=False) -> "
         "(Tensor, Tensor, Tensor, Tensor, Tensor)");
@@ -673,6 +802,8 @@ TORCH_LIBRARY_IMPL(pnfx, CUDA, m) {
   m.impl("linear_wgrad", linear_wgrad_cuda);
   m.impl("flash_fwd", flash_fwd_cuda);
   m.impl("flash_bwd", flash_bwd_cuda);
+  m.impl("attn_rows", attn_rows_cuda);
+  m.impl("attn_rows_bwd", attn_rows_bwd_cuda);
   m.impl("flash_fwd_fir", flash_fwd_fir_cuda);
 }
 
@@ -680,5 +811,6 @@ TORCH_LIBRARY_IMPL(pnfx, Autograd, m) {
   m.impl("fir_fwd", fir_fwd_autograd);
   m.impl("pn_rows_fwd", pn_rows_fwd_autograd);
   m.impl("linear", linear_autograd);
+  m.impl("attn_rows", attn_rows_autograd);
   m.impl("flash_fwd", flash_fwd_autograd);
 }

@@ -187,6 +187,30 @@ def fused_fir_forward_applies(q: torch.Tensor, k_raw: torch.Tensor, taps: torch.
                                               or taps.requires_grad))
 
 
+def attn_rows_applies(qkv: torch.Tensor, taps: torch.Tensor, n_heads: int) -> bool:
+    """Whether PnFirTauFlashMHA's training forward may run pnfx::attn_rows on its projection rows
+    [B, N, 3 D]: the same two kernels forward and the same stages backward, with the same bits, as
+    hip_causal_fir and the flash op on the split rows, without the copy that joins the gradients of
+    q, k and v (19 of 383 us of GPU time at B=32 N=512 D=256) and the dozen view nodes of the split.
+    bf16 rows that reach the kernels as they are: contiguous, 7 taps, head sizes in whole 16-byte
+    chunks up to FLASH_MAX_HEAD_DIM."""
+    D = qkv.shape[-1] // 3
+    return (torch.is_grad_enabled() and qkv.requires_grad and qkv.is_cuda
+            and qkv.dtype == torch.bfloat16 and qkv.dim() == 3 and qkv.is_contiguous()
+            and qkv.numel() > 0 and taps.numel() == FIR_KERNEL_TAPS and D <= FIR_KERNEL_MAX_C
+            and (D // n_heads) % 8 == 0 and D // n_heads <= FLASH_MAX_HEAD_DIM
+            and qkv.data_ptr() % 16 == 0 and not taps.requires_grad
+            and torch._C._functorch.peek_interpreter_stack() is None)
+
+
+def attn_rows(qkv, taps, score_tau, n_heads, scale, gamma, causal_mask):
+    """O [B, N, D] of the key FIR and flash attention over projection rows [B, N, 3 D]."""
+    has_gamma = gamma is not None and gamma > 0.0
+    return torch.ops.pnfx.attn_rows.default(qkv, taps.reshape(-1), score_tau, n_heads,
+                                            float(scale), float(gamma) if has_gamma else 0.0,
+                                            has_gamma, bool(causal_mask))[0]
+
+
 def fused_fir_flash_forward(q, k_raw, v, taps, score_tau, scale, gamma, causal_mask):
     """O [B, H, N, d] (backed by [B, N, H, d] memory) of the flash forward with the causal FIR of
     the raw keys fused into its key-tile load: bitwise hip_causal_fir followed by

@@ -167,6 +167,20 @@ def _(q, k, v, tau, o, o_lo, do, M, Z, mask, scale, gamma, has_gamma, causal):
     return _grad_like(q), _grad_like(k), _grad_like(v), q.new_empty(1, dtype=torch.float32)
 
 
+@torch.library.register_fake("pnfx::attn_rows")
+def _(qkv, taps, tau, heads, scale, gamma, has_gamma, causal):
+    B, N, C = qkv.shape[0], qkv.shape[1], qkv.shape[2] // 3
+    f = lambda: qkv.new_empty((B, heads, N), dtype=torch.float32)  # noqa: E731
+    o_lo = qkv.new_empty((B, N, heads, C // heads)).permute(0, 2, 1, 3)
+    return (qkv.new_empty((B, N, C)), o_lo, qkv.new_empty((B, N, C)), f(), f(),
+            qkv.new_empty(_mask_shape(B, heads, N), dtype=torch.uint8))
+
+
+@torch.library.register_fake("pnfx::attn_rows_bwd")
+def _(qkv, k, taps, tau, o, o_lo, do, M, Z, mask, scale, gamma, has_gamma, causal):
+    return qkv.new_empty(qkv.shape), qkv.new_empty(1, dtype=torch.float32)
+
+
 @torch.library.register_fake("pnfx::flash_fwd_fir")
 def _(q, k_raw, v, tau, taps, scale, gamma, has_gamma, causal, o_bnhd=False):
     _check_qkv(q, k_raw, v)

@@ -200,7 +200,13 @@ class PnFirTauFlashMHA(PnFirTauMHA):
 
         cfg = self.cfg
         B, N, D = x.shape
-        q, k_raw, v = hp.project(self.qkv, x).split(D, dim=-1)
+        qkv = hp.project(self.qkv, x)
+        if not torch.compiler.is_compiling() and hp.attn_rows_applies(qkv, self.fir_taps,
+                                                                      self.n_heads):
+            o = hp.attn_rows(qkv, self.fir_taps, self.score_tau, self.n_heads,
+                             1.0 / math.sqrt(self.head_dim), cfg.silence_gamma, cfg.causal_mask)
+            return hp.project(self.out, o)
+        q, k_raw, v = qkv.split(D, dim=-1)
         if hp.fused_fir_forward_applies(q, k_raw, self.fir_taps, self.head_dim):
             # inference: the key FIR inside the forward's key-tile load (one launch, same bits)
             o = hp.fused_fir_flash_forward(self._split_heads(q), self._split_heads(k_raw),

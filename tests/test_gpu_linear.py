@@ -87,3 +87,22 @@ def test_project_keeps_hooks_and_second_order(dev, monkeypatch):
     assert calls == [1]
     for a, b in zip(got, ref):
         assert (a - b).float().norm() <= 2.0 ** -6 * b.float().norm()
+
+
+@pytest.mark.parametrize("B,N,D,H", [(2, 70, 64, 4), (1, 129, 240, 3), (3, 33, 128, 1), (1, 1, 16, 2)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_attn_rows_is_the_split_path(dev, monkeypatch, B, N, D, H, causal):
+    """The module on projection rows: bitwise the FIR and flash ops on the split rows."""
+    print(f"[attn_rows B={B} N={N} D={D} H={H} causal={causal}]", flush=True)
+    torch.manual_seed(1)
+    m = PnFirTauFlashMHA(PnFirConfig(d_model=D, n_heads=H, causal_mask=causal, tau_init=0.05)).to(dev)
+    x = seeded((B, N, D), 7, torch.float32, dev).requires_grad_()
+    dy = seeded((B, N, D), 8, torch.bfloat16, dev)
+    calls = []
+    rows = hip_pnfirtau.attn_rows
+    monkeypatch.setattr(hip_pnfirtau, "attn_rows", lambda *a: (calls.append(1), rows(*a))[1])
+    got = _grads(m, x, dy, True)
+    assert calls == [1]
+    monkeypatch.setattr(hip_pnfirtau, "attn_rows_applies", lambda *a: False)
+    for a, b in zip(got, _grads(m, x, dy, True)):
+        assert a.dtype == b.dtype and torch.equal(a, b)
