@@ -138,6 +138,7 @@ int pnfx_linear_wgrad(const void* dy, int64_t dy_rs, const void* x, int64_t x_rs
  *                1 where the 32-query x 64-key sub-tile has a positive
  *                rectified score (the skip rule of src/triton_pnfirtau.py:395-400
  *                at 32-row granularity; OR adjacent row pairs for the 64x64 view).
+ *                fp32: N <= 65536 with a mask (PNFX_EINVAL above it; pass NULL there).
  *   workspace  : optional (may be NULL), pnfx_flash_fwd_workspace_size(B, H, N, D)
  *                bytes, 256-byte aligned.  With it (bf16, tau > 0) the forward first
  *                takes the largest key norm of every 64-key tile and skips, without

@@ -105,6 +105,10 @@ struct BwdWorkspace {
   static int64_t round256(int64_t x) { return (x + 255) / 256 * 256; }
 };
 
+// Longest sequence whose tile mask the fp32 forward can form (it and the dQ kernel keep one entry per
+// 64-key tile in LDS).
+constexpr int64_t kF32MaskMaxN = 65536;
+
 int flash_fwd_bf16(const FwdParams& fp, int64_t D, bool causal, hipStream_t st);
 // Rows of fp.d columns, fp.d a multiple of 8 without a kernel of its own.
 int flash_fwd_ragged_bf16(const FwdParams& fp, bool causal, hipStream_t st);

@@ -111,6 +111,10 @@ static int flash_fwd_impl(bool any, const void* q, int64_t qsb, int64_t qsh, int
   PNFX_REQUIRE(M && Z && tau, "flash_fwd: null statistics / tau pointer");
   PNFX_REQUIRE(!o_lo || (dtype == PNFX_BF16 && aligned16(o_lo)),
                "flash_fwd: o_lo is a 16-byte aligned bf16 buffer with o's strides");
+  // the fp32 forward holds one activity bit per key tile in LDS, for 1024 tiles
+  PNFX_REQUIRE(!tile_mask || dtype == PNFX_BF16 || N <= kF32MaskMaxN,
+               "flash_fwd: fp32 tile_mask at N=%lld (up to %lld)", (long long)N,
+               (long long)kF32MaskMaxN);
   const int64_t fws = pnfx_flash_fwd_workspace_size(B, H, N, D);
   PNFX_REQUIRE(!workspace || (workspace_bytes >= fws &&
                               (reinterpret_cast<uintptr_t>(workspace) & 255u) == 0),

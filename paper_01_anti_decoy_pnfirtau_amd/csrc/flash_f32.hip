@@ -67,8 +67,8 @@ template <>
 struct Score<false> { typedef float type; };
 template <int D>
 using score_t = typename Score<(D <= 64)>::type;
-// Key tiles of one sequence with a tile mask (N <= 65536, the mask's own limit)
-constexpr int kMaxTiles = 1024;
+// Key tiles of one sequence with a tile mask
+constexpr int kMaxTiles = kF32MaskMaxN / TB;
 
 __device__ __forceinline__ float pow10f_(float u) {
   const float u2 = u * u;

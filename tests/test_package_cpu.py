@@ -159,6 +159,17 @@ def test_c_abi_rejects_bad_arguments_without_touching_the_gpu():
     assert rc == -1 and b"bf16 only" in lib.pnfx_last_error()
 
 
+def test_fp32_forward_refuses_a_tile_mask_past_its_length_limit():
+    """The fp32 forward keeps an activity bit per key tile in LDS for sequences up to 65536: a tile
+    mask past that is refused on the host, before any device call."""
+    lib = _lib.lib()
+    fake = ctypes.c_void_p(256)
+    N = 65536 + 1
+    args = [fake, 16 * N, 16 * N, 16] * 4 + [None, fake, fake, None, fake, None, 0, 1, 1, N, 16,
+                                             fake, 0.25, 0.5, 1, 1, _lib.PNFX_F32, None]
+    assert lib.pnfx_flash_fwd(*args) == -1 and b"tile_mask at N=65537" in lib.pnfx_last_error()
+
+
 @pytest.mark.parametrize("B,H,N,D", [(4, 16, 8192, 64), (8, 8, 4096, 128), (1, 3, 520, 128),
                                      (2, 4, 1000, 32), (1, 1, 70000, 16)])
 def test_backward_workspace_holds_only_what_the_kernels_use(B, H, N, D):
