@@ -553,14 +553,15 @@ Tensor fir_fwd_autograd(const Tensor& x, const Tensor& taps) {
 }
 
 // x W^T for bf16 rows x and a bf16 or fp32 weight without bias, with the weight gradient from
-// pnfx_linear_wgrad in W's own type.
+// pnfx_linear_wgrad in W's own type.  wb is W's bf16 copy, made by autograd's own cast: the product
+// and its gradients use the copy, which a later change of W does not reach, and a differentiable
+// backward follows it to W.
 class LinearFn : public torch::autograd::Function<LinearFn> {
  public:
-  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, const Tensor& wb) {
     at::AutoDispatchBelowADInplaceOrView guard;
-    const Tensor wb = w.to(at::kBFloat16);
     ctx->save_for_backward({x, wb});
-    ctx->saved_data["w"] = w;  // for a differentiable backward only
+    ctx->saved_data["wide"] = w.scalar_type() == at::kFloat;
     return linear_op().call(x, wb);
   }
   static const c10::TypedOperatorHandle<Tensor(const Tensor&, const Tensor&)>& linear_op() {
@@ -570,17 +571,19 @@ class LinearFn : public torch::autograd::Function<LinearFn> {
   static variable_list backward(AutogradContext* ctx, variable_list gy) {
     static auto wgrad =
         op("pnfx::linear_wgrad").typed<Tensor(const Tensor&, const Tensor&, bool)>();
-    variable_list out(2);
+    variable_list out(3);
     if (!gy[0].defined()) return out;
     const auto s = ctx->get_saved_variables();
-    const Tensor w = ctx->saved_data["w"].toTensor();
-    const bool again = at::GradMode::is_enabled();  // create_graph: products autograd can follow
-    const Tensor wb = again ? w.to(at::kBFloat16) : s[1];
-    const Tensor g2 = gy[0].reshape({-1, w.size(0)}), x2 = s[0].reshape({-1, w.size(1)});
-    if (ctx->needs_input_grad(0)) out[0] = at::mm(g2, wb).view(s[0].sizes());
-    if (ctx->needs_input_grad(1))
-      out[1] = again ? at::mm(g2.t(), x2).to(w.scalar_type())
-                     : wgrad.call(g2, x2, w.scalar_type() == at::kFloat);
+    const Tensor &x = s[0], &wb = s[1];
+    const bool wide = ctx->saved_data["wide"].toBool();
+    const Tensor g2 = gy[0].reshape({-1, wb.size(0)}), x2 = x.reshape({-1, wb.size(1)});
+    if (ctx->needs_input_grad(0)) out[0] = at::mm(g2, wb).view(x.sizes());
+    if (ctx->needs_input_grad(1)) {
+      if (at::GradMode::is_enabled())  // create_graph: products that autograd can follow
+        out[1] = at::mm(g2.t(), x2).to(wide ? at::kFloat : at::kBFloat16);
+      else
+        out[1] = wgrad.call(g2, x2, wide);
+    }
     return out;
   }
 };
@@ -590,7 +593,7 @@ Tensor linear_autograd(const Tensor& x, const Tensor& w) {
     at::AutoDispatchBelowADInplaceOrView guard;
     return LinearFn::linear_op().call(x, w);
   }
-  return LinearFn::apply(x, w);
+  return LinearFn::apply(x, w, w.to(at::kBFloat16));
 }
 
 const auto& rows_fwd_op() {

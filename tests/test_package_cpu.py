@@ -201,6 +201,43 @@ def test_hip_ops_refuse_cpu_tensors():
         P.flash_pn_fir_tau_attention(q, q, q, torch.tensor(0.0))
 
 
+@pytest.mark.parametrize("wdtype", [torch.float32, torch.bfloat16])
+def test_linear_op_gradients_are_those_of_the_library_linear(wdtype):
+    """pnfx::linear's autograd (its kernels stood in for on the CPU): first and second order as
+    F.linear on the weight's bf16 copy, and an fp32 weight that changes between forward and backward
+    (an optimizer step) leaves both orders those of the weight that the forward used."""
+    from paper_01_anti_decoy_pnfirtau_amd import ops  # noqa: F401
+
+    g = torch.Generator().manual_seed(3)
+    w0 = torch.randn(16, 24, generator=g).to(wdtype)
+    x0, gy = (torch.randn(8, n, generator=g).bfloat16() for n in (24, 16))
+
+    def grads(linear, create_graph, change):
+        x, w = x0.clone().requires_grad_(), w0.clone().requires_grad_()
+        y = linear(x, w)
+        if change:
+            with torch.no_grad():
+                w.mul_(3.0)
+        first = torch.autograd.grad(y, [x, w], y.detach() + gy, create_graph=create_graph)
+        if not create_graph:
+            return first
+        second = torch.autograd.grad(sum(t.float().square().sum() for t in first), [x, w])
+        return (*first, *second)
+
+    with torch.library._scoped_library("pnfx", "IMPL") as lib:
+        lib.impl("linear", lambda x, w: x @ w.to(x.dtype).t(), "CPU")
+        lib.impl("linear_wgrad", lambda dy, x, wide: (dy.float().t() @ x.float()).to(
+            torch.float32 if wide else dy.dtype), "CPU")
+        for create_graph in (False, True):
+            for change in ((False, True) if wdtype == torch.float32 else (False,)):
+                got = grads(torch.ops.pnfx.linear.default, create_graph, change)
+                ref = grads(lambda x, w: torch.nn.functional.linear(x, w.bfloat16()), create_graph,
+                            change)
+                for a, b in zip(got, ref):  # roundings to bf16 of the products and their sums
+                    assert a.dtype == b.dtype
+                    assert (a - b).float().norm() <= 2.0 ** -6 * b.float().norm()
+
+
 def test_wikilm_variants_share_init_and_train_on_cpu():
     """The LM consumer (experiments/exp4_wikitext2_lm.py:183-247) builds the same weights for
     every attention variant from one seed and ties the head to the embedding.  Off-GPU the
