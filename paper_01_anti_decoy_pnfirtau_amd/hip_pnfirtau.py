@@ -86,6 +86,9 @@ def hip_pn_fir_tau_scores(
     return w
 
 
+PLAIN = (torch.Tensor, torch.nn.Parameter)  # neither a subclass nor a stand-in without memory
+
+
 def split_wgrad_applies(rows: int, out_features: int, in_features: int) -> bool:
     """Whether pnfx::linear_wgrad is the faster weight gradient: many rows over a small weight, where
     one workgroup per output tile leaves the chip idle.  Measured on MI355X (us, this kernel against
@@ -115,8 +118,7 @@ def project(lin: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
              or lin._backward_pre_hooks or "forward" in lin.__dict__
              or nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks
              or nn_module._global_backward_hooks or nn_module._global_backward_pre_hooks)
-    plain = (torch.Tensor, torch.nn.Parameter)
-    if (not bf16 or hooks or type(w) not in plain or type(x) not in plain or x.dim() < 2
+    if (not bf16 or hooks or type(w) not in PLAIN or type(x) not in PLAIN or x.dim() < 2
             or x.shape[-1] != w.shape[1] or w.device != x.device
             or torch._C._functorch.peek_interpreter_stack() is not None
             or not split_wgrad_applies(x.numel() // max(1, x.shape[-1]), *w.shape)):
@@ -193,9 +195,9 @@ def attn_rows_applies(qkv: torch.Tensor, taps: torch.Tensor, n_heads: int) -> bo
     hip_causal_fir and the flash op on the split rows, without the copy that joins the gradients of
     q, k and v (19 of 383 us of GPU time at B=32 N=512 D=256) and the dozen view nodes of the split.
     bf16 rows that reach the kernels as they are: contiguous, 7 taps, head sizes in whole 16-byte
-    chunks up to FLASH_MAX_HEAD_DIM."""
+    chunks up to FLASH_MAX_HEAD_DIM; of a plain tensor (a fake or functional one has no address)."""
     D = qkv.shape[-1] // 3
-    return (torch.is_grad_enabled() and qkv.requires_grad and qkv.is_cuda
+    return (type(qkv) in PLAIN and torch.is_grad_enabled() and qkv.requires_grad and qkv.is_cuda
             and qkv.dtype == torch.bfloat16 and qkv.dim() == 3 and qkv.is_contiguous()
             and qkv.numel() > 0 and taps.numel() == FIR_KERNEL_TAPS and D <= FIR_KERNEL_MAX_C
             and (D // n_heads) % 8 == 0 and D // n_heads <= FLASH_MAX_HEAD_DIM

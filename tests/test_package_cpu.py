@@ -325,6 +325,30 @@ def test_fake_kernels_give_the_output_layouts():
         assert d_raw.shape == raw.shape and dtr.shape == (B * H * N,)
 
 
+@pytest.mark.filterwarnings("error::UserWarning")
+def test_flash_module_training_forward_traces_on_fake_and_functional_tensors(monkeypatch):
+    """The module's training forward on tensors without an address (shape runs, tracing without
+    Dynamo): the split path, the output's shape, and no look at a data pointer."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch._subclasses.functional_tensor import FunctionalTensor, FunctionalTensorMode
+
+    from paper_01_anti_decoy_pnfirtau_amd import hip_pnfirtau
+
+    monkeypatch.setattr(hip_pnfirtau, "attn_rows", None)
+    with FakeTensorMode():
+        with torch.device("cuda"):
+            m = P.PnFirTauFlashMHA(P.PnFirConfig(d_model=64, n_heads=4))
+            for lin in (m.qkv, m.out):
+                lin.weight = torch.nn.Parameter(torch.empty(lin.weight.shape, dtype=torch.bfloat16))
+            x = torch.empty(2, 40, 64, dtype=torch.bfloat16)
+        x.requires_grad_()
+        y = m(x)
+        assert y.shape == x.shape and y.requires_grad
+        with FunctionalTensorMode():
+            yf = m(FunctionalTensor.to_functional(x))
+            assert yf.shape == x.shape and type(yf) is FunctionalTensor
+
+
 def test_tile_mask_shape_and_its_length_limit():
     """The forward's silence map is [B*H, ceil(N/32), ceil(N/64)] bytes -- N^2/2048 per (b, h) --
     and is not formed past MASK_MAX_N (the backward then recomputes every tile)."""
