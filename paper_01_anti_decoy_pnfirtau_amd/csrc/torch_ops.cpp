@@ -434,7 +434,8 @@ void check_qkv_rows(const Tensor& qkv, const Tensor& taps, int64_t H) {
                     "attn_rows: head dim ", qkv.size(2) / (3 * H), ", taps ", taps.sizes());
 }
 
-// o rows [B, N, H d], o_lo [B, H, N, d] over such rows, the filtered key rows, M, Z, tile mask
+// o and o_lo as rows [B, N, H d], the filtered key rows, M, Z, tile mask.  (Rows, so that a saved-tensor
+// hook that lays o and o_lo out anew leaves them alike: the backward drops a residual of other strides.)
 std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> attn_rows_cuda(
     const Tensor& qkv, const Tensor& taps, const Tensor& tau, int64_t H, double scale,
     double gamma, bool has_gamma, bool causal) {
@@ -444,7 +445,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> attn_rows_cuda(
   auto [o, o_lo, M, Z, Nm, mask] = flash_fwd_cuda(
       rows_as_heads(qkv.narrow(2, 0, C), H), rows_as_heads(kf, H),
       rows_as_heads(qkv.narrow(2, 2 * C, C), H), tau, scale, gamma, has_gamma, causal, true, false);
-  return {o.transpose(1, 2).view({qkv.size(0), qkv.size(1), C}), o_lo, kf, M, Z, mask};
+  const auto as_rows = [&](const Tensor& t) {
+    return t.transpose(1, 2).view({qkv.size(0), qkv.size(1), C});
+  };
+  return {as_rows(o), as_rows(o_lo), kf, M, Z, mask};
 }
 
 std::tuple<Tensor, Tensor> attn_rows_bwd_cuda(
@@ -453,14 +457,15 @@ std::tuple<Tensor, Tensor> attn_rows_bwd_cuda(
     double scale, double gamma, bool has_gamma, bool causal) {
   const int64_t H = M.size(1), C = qkv.size(2) / 3;
   check_qkv_rows(qkv, taps, H);
-  TORCH_CHECK_VALUE(dout.sizes() == o.sizes(), "attn_rows_bwd: dO has shape ", dout.sizes(),
-                    ", O ", o.sizes());
+  TORCH_CHECK_VALUE(dout.sizes() == o.sizes() && o_lo.sizes() == o.sizes(),
+                    "attn_rows_bwd: dO has shape ", dout.sizes(), ", O ", o.sizes(),
+                    ", its residual ", o_lo.sizes());
   const c10::DeviceGuard guard(qkv.device());
   Tensor d = at::empty(qkv.sizes(), qkv.options());
   const Tensor dk_raw = d.narrow(2, C, C);
   const auto heads = [&](int64_t i) { return rows_as_heads(qkv.narrow(2, i * C, C), H); };
   auto [dq, dk, dv, dtau] = flash_bwd_into(
-      heads(0), rows_as_heads(kf, H), heads(2), tau, rows_as_heads(o, H), o_lo,
+      heads(0), rows_as_heads(kf, H), heads(2), tau, rows_as_heads(o, H), rows_as_heads(o_lo, H),
       rows_as_heads(dout.contiguous(), H), M, Z, mask, scale, gamma, has_gamma, causal,
       {rows_as_heads(d.narrow(2, 0, C), H), Tensor(), rows_as_heads(d.narrow(2, 2 * C, C), H)});
   const Tensor t = taps.to(qkv.device(), at::kFloat).contiguous();

@@ -171,8 +171,7 @@ def _(q, k, v, tau, o, o_lo, do, M, Z, mask, scale, gamma, has_gamma, causal):
 def _(qkv, taps, tau, heads, scale, gamma, has_gamma, causal):
     B, N, C = qkv.shape[0], qkv.shape[1], qkv.shape[2] // 3
     f = lambda: qkv.new_empty((B, heads, N), dtype=torch.float32)  # noqa: E731
-    o_lo = qkv.new_empty((B, N, heads, C // heads)).permute(0, 2, 1, 3)
-    return (qkv.new_empty((B, N, C)), o_lo, qkv.new_empty((B, N, C)), f(), f(),
+    return (qkv.new_empty((B, N, C)), qkv.new_empty((B, N, C)), qkv.new_empty((B, N, C)), f(), f(),
             qkv.new_empty(_mask_shape(B, heads, N), dtype=torch.uint8))
 
 

@@ -106,3 +106,19 @@ def test_attn_rows_is_the_split_path(dev, monkeypatch, B, N, D, H, causal):
     monkeypatch.setattr(hip_pnfirtau, "attn_rows_applies", lambda *a: False)
     for a, b in zip(got, _grads(m, x, dy, True)):
         assert a.dtype == b.dtype and torch.equal(a, b)
+
+
+def test_attn_rows_under_saved_tensor_hooks(dev):
+    """Saved tensors that come back freshly laid out (offloading to pinned host memory): the same
+    gradients, O's rounding residual among what the backward uses."""
+    torch.manual_seed(2)
+    m = PnFirTauFlashMHA(PnFirConfig(d_model=64, n_heads=4, tau_init=0.05)).to(dev)
+    x = seeded((2, 150, 64), 9, torch.float32, dev).requires_grad_()
+    dy = seeded((2, 150, 64), 10, torch.bfloat16, dev)
+    ref = _grads(m, x, dy, True)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: torch.empty(t.shape, dtype=t.dtype,
+                                                                        device=dev).copy_(t),
+                                                  lambda t: t):
+        got = _grads(m, x, dy, True)
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b)
