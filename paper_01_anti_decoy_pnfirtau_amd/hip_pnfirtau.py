@@ -95,9 +95,10 @@ def split_wgrad_applies(rows: int, out_features: int, in_features: int) -> bool:
     the library product and its cast to fp32): 768x256 over 16384 rows 29 / 93, over 2048 12 / 17,
     over 512 9.8 / 10.0; 1536x512 over 8192 42 / 55, over 2048 24 / 19; 768x768 over 8192 36 / 51,
     over 2048 22 / 18; 1024x1024 over 8192 34 / 56; 2304x768 over 16384 127 / 124; 3072x1024 over
-    65536 1272 / 492.  Columns in whole 16-byte chunks."""
+    65536 1272 / 492.  Columns in whole 16-byte chunks; sizes that the kernel's entry takes."""
     mn = out_features * in_features
-    return out_features % 8 == 0 and in_features % 8 == 0 and mn <= 128 * rows and mn <= 1 << 20
+    return (out_features % 8 == 0 and in_features % 8 == 0 and mn <= 128 * rows and mn <= 1 << 20
+            and max(out_features, in_features) <= 65536 and rows < 1 << 30)
 
 
 def project(lin: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
