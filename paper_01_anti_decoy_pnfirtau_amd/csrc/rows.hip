@@ -314,11 +314,12 @@ __global__ __launch_bounds__(256, CH == 1 ? 8 : CH == 2 ? 6 : 4) void pn_rows_bw
 
   float u[CH][V], dy[CH][V];
   float dot = 0.0f;
-  const auto add_dot = [&](const float (&uc)[V], const float (&g)[V]) {
+  // only the chunk's first nv entries of dW: one past the causal limit may be an infinity
+  const auto add_dot = [&](const float (&uc)[V], const float (&g)[V], int nv) {
 #pragma unroll
     for (int j = 0; j < V; ++j) {
       const float pw = pow_p<PMODE>(uc[j], a.p);
-      dot = __builtin_fmaf(g[j], PMODE ? pw : pw / z, dot);
+      dot = __builtin_fmaf(j < nv ? g[j] : 0.0f, PMODE ? pw : pw / z, dot);
     }
   };
 #pragma unroll
@@ -330,18 +331,20 @@ __global__ __launch_bounds__(256, CH == 1 ? 8 : CH == 2 ? 6 : 4) void pn_rows_bw
       load_chunk<T, ANY>(row, c0, a.N, x);
       load_chunk<T, ANY>(dyrow, c0, a.N, g);
     }
-    rectify(x, scale, ntau, valid_in_chunk(limit, c0), u[k]);
+    const int nv = valid_in_chunk(limit, c0);
+    rectify(x, scale, ntau, nv, u[k]);
 #pragma unroll
     for (int j = 0; j < V; ++j) dy[k][j] = g[j];
-    add_dot(u[k], g);
+    add_dot(u[k], g, nv);
   }
   for (int64_t c0 = CH * SPAN + cl; c0 - cl < limit; c0 += SPAN) {
     if (c0 >= limit) continue;
     float x[V], g[V], uc[V];
     load_chunk<T, ANY>(row, c0, a.N, x);
     load_chunk<T, ANY>(dyrow, c0, a.N, g);
-    rectify(x, scale, ntau, valid_in_chunk(limit, c0), uc);
-    add_dot(uc, g);
+    const int nv = valid_in_chunk(limit, c0);
+    rectify(x, scale, ntau, nv, uc);
+    add_dot(uc, g, nv);
   }
   dot = row_sum(dot);
   if (PMODE) dot /= z;

@@ -132,3 +132,20 @@ def test_sum_f64_is_the_double_sum(dev, n):
         assert abs(float(torch.ops.pnfx.sum_f64(t, True)) - want) <= bound
         got = torch.ops.pnfx.sum_f64(t, False)
         assert got.dtype == torch.float32 and abs(float(got) - want) <= 6e-8 * abs(want) + bound
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N", [31, 64, 777, 2100])
+def test_rows_masked_weight_gradients_reach_nothing(dev, dtype, N):
+    """Infinities and NaN of dW past the causal limit, in the 16-byte chunk that straddles it and after
+    it: the gradients of the same call with zeros there, bit for bit."""
+    raw = seeded((1, 1, N, N), 35, dtype, dev, scale=2.0)
+    dW = seeded((1, 1, N, N), 36, dtype, dev).tril_()
+    bad = torch.full_like(dW, float("inf"))
+    bad[..., 1::2] = float("nan")
+    tau = torch.tensor(0.1, device=dev)
+    for p in (10.0, 2.0, 3.5):
+        w, M, Z, Nm = torch.ops.pnfx.pn_rows_fwd(raw, tau, 0.5, p, 0.5, True, True)
+        want = torch.ops.pnfx.pn_rows_bwd(dW, raw, tau, M, Z, Nm, 0.5, p, 0.5, True, True)
+        got = torch.ops.pnfx.pn_rows_bwd(dW + bad.triu(1), raw, tau, M, Z, Nm, 0.5, p, 0.5, True, True)
+        assert all(torch.equal(a, b) and torch.isfinite(a).all() for a, b in zip(got, want)), p
