@@ -347,7 +347,12 @@ __global__ __launch_bounds__(256, CH == 1 ? 8 : CH == 2 ? 6 : 4) void pn_rows_bw
     add_dot(uc, g, nv);
   }
   dot = row_sum(dot);
-  if (PMODE) dot /= z;
+  if (PMODE) {
+    dot /= z;
+    // A power of the forward overflowed: its W held inf * 0, and no entry has a gradient (the
+    // unit's powers are finite, so the sum alone would end as 0).
+    if (pow_p<PMODE>(peak, a.p) == __builtin_inff()) dot = __builtin_nanf("");
+  }
 
   float gate = 1.0f, gterm = 0.0f;
   if (a.has_gamma) {

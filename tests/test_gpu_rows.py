@@ -149,3 +149,28 @@ def test_rows_masked_weight_gradients_reach_nothing(dev, dtype, N):
         want = torch.ops.pnfx.pn_rows_bwd(dW, raw, tau, M, Z, Nm, 0.5, p, 0.5, True, True)
         got = torch.ops.pnfx.pn_rows_bwd(dW + bad.triu(1), raw, tau, M, Z, Nm, 0.5, p, 0.5, True, True)
         assert all(torch.equal(a, b) and torch.isfinite(a).all() for a, b in zip(got, want)), p
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("p,big", [(10.0, 1e4), (2.0, 1e20), (3.5, 1e12)])
+@pytest.mark.parametrize("N", [64, 95])
+def test_rows_overflow_of_the_powers_stays_visible(dev, dtype, p, big, N):
+    """A row whose largest score's power overflows fp32 has NaN in W, and NaN for the gradient of each
+    of its positive scores and of tau, not zeros; the other rows are those of the call without it."""
+    raw = seeded((1, 1, N, N), 37, dtype, dev)
+    dW = seeded((1, 1, N, N), 38, dtype, dev)
+    tau = torch.tensor(0.0, device=dev)
+    res = []
+    for spike in (None, big):
+        r = raw.clone()
+        if spike:
+            r[0, 0, 40, 7] = spike
+        w, M, Z, Nm = torch.ops.pnfx.pn_rows_fwd(r, tau, 1.0, p, 0.5, True, True)
+        d, dt = torch.ops.pnfx.pn_rows_bwd(dW, r, tau, M, Z, Nm, 1.0, p, 0.5, True, True)
+        res.append((w[0, 0], d[0, 0], dt, r[0, 0]))
+    (w0, d0, t0, _), (w, d, t, r) = res
+    others = torch.arange(N, device=dev) != 40
+    assert all(torch.equal(a[others], b[others]) for a, b in ((w, w0), (d, d0), (t, t0)))
+    on = (r[40] > 0) & (torch.arange(N, device=dev) <= 40)
+    assert torch.isnan(w[40, 7]) and torch.isnan(t[40])
+    assert torch.equal(torch.isnan(d[40]), on) and bool((d[40][~on] == 0).all())
