@@ -163,19 +163,14 @@ __device__ __forceinline__ void rectify(const float (&x)[V], float scale, float 
     u[j] = j < nv ? s : 0.0f;
   }
 }
-// dW past a chunk's first nv entries, where it may be an infinity: 0.  (A branch: few chunks straddle
-// the limit, and a select in each cost the backward 10 % for p = 3.5.)
-template <int V>
-__device__ __forceinline__ void drop_masked(int nv, float (&g)[V]) {
-  if (nv < V) {
-#pragma unroll
-    for (int j = 0; j < V; ++j) g[j] = j < nv ? g[j] : 0.0f;
-  }
-}
 __device__ __forceinline__ int valid_in_chunk(int64_t limit, int64_t c0) {
   const int64_t n = limit - c0;
   return n < 0 ? 0 : n > 16 ? 16 : (int)n;
 }
+
+// Chunks held in registers by the kernels of the longest rows (shorter rows have a kernel that holds
+// all of theirs).
+constexpr int kMaxChunks = 4;
 
 // Lane l owns columns [l*V, l*V + V) of every 64*V-column chunk.  The first CH chunks of a
 // row stay in registers between the two passes (u, and dW in the backward); columns beyond
@@ -190,6 +185,7 @@ template <typename T, int PMODE, bool ANY, int CH>
 __global__ __launch_bounds__(256, CH <= 2 ? 8 : 4) void pn_rows_fwd_kernel(RowsArgs a) {
   constexpr int V = RowIO<T, ANY>::V;
   constexpr int64_t SPAN = 64 * V;
+  constexpr bool MORE = CH == kMaxChunks;  // rows longer than the registers
   const int64_t r = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (r >= a.R) return;
@@ -221,7 +217,7 @@ __global__ __launch_bounds__(256, CH <= 2 ? 8 : 4) void pn_rows_fwd_kernel(RowsA
       mass += pu;
     }
   }
-  for (int64_t c0 = CH * SPAN + cl; c0 - cl < limit; c0 += SPAN) {
+  for (int64_t c0 = CH * SPAN + cl; MORE && c0 - cl < limit; c0 += SPAN) {
     if (c0 >= limit) continue;
     float x[V], uc[V];
     load_chunk<T, ANY>(row, c0, a.N, x);
@@ -263,7 +259,7 @@ __global__ __launch_bounds__(256, CH <= 2 ? 8 : 4) void pn_rows_fwd_kernel(RowsA
     }
     if (c0 < a.N) store_chunk<T, ANY>(wrow, c0, a.N, w);
   }
-  for (int64_t c0 = CH * SPAN + cl; c0 - cl < a.N; c0 += SPAN) {
+  for (int64_t c0 = CH * SPAN + cl; MORE && c0 - cl < a.N; c0 += SPAN) {
     if (c0 >= a.N) continue;
     float w[V] = {};
     if (c0 < limit) {
@@ -297,6 +293,23 @@ __device__ __forceinline__ float pow_pm1(float u) {
   }
 }
 
+// <dW, w_hat> of a row entry by entry over its valid columns, for rows where the backward's own sum
+// does not tell: it is NaN (a chunk's dW past the causal limit may be an infinity, times a power of 0),
+// or a power overflowed in the forward (inf / inf here; the backward's unit would end as 0).  A test
+// of each entry instead cost the backward 5-10 % (17.2 -> 18.1 us at [64, 1, 512, 512] bf16).
+template <typename T, int PMODE>
+__device__ __forceinline__ float plain_dot(const RowsArgs& a, const T* row, const T* dyrow,
+                                           int64_t limit, int lane, float z) {
+  const float ntau = -a.tau[0];
+  float dot = 0.0f;
+#pragma unroll 1
+  for (int64_t c = lane; c < limit; c += 64) {
+    const float u = fmaxf(__builtin_fmaf(to_f32(row[c]), a.scale, ntau), 0.0f);
+    dot = __builtin_fmaf(to_f32(dyrow[c]), pow_p<PMODE>(u, a.p) / z, dot);
+  }
+  return row_sum(dot);
+}
+
 // The backward takes the scores in units of the power of two of the row's peak for p = 10 and 2
 // (an exact scaling, folded into scale and tau): the powers are then at most 1, so that the sum
 // <dW, u^p> can be divided by Z once instead of entry by entry without overflowing.  Peaks below
@@ -305,6 +318,7 @@ template <typename T, int PMODE, bool ANY, int CH>
 __global__ __launch_bounds__(256, CH == 1 ? 8 : CH == 2 ? (PMODE ? 6 : 5) : PMODE ? 4 : 3) void pn_rows_bwd_kernel(RowsArgs a) {
   constexpr int V = RowIO<T, ANY>::V;
   constexpr int64_t SPAN = 64 * V;
+  constexpr bool MORE = CH == kMaxChunks;  // rows longer than the registers
   const int64_t r = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (r >= a.R) return;
@@ -347,30 +361,23 @@ __global__ __launch_bounds__(256, CH == 1 ? 8 : CH == 2 ? (PMODE ? 6 : 5) : PMOD
       load_chunk<T, ANY>(row, c0, a.N, x);
       load_chunk<T, ANY>(dyrow, c0, a.N, g);
     }
-    const int nv = valid_in_chunk(limit, c0);
-    rectify(x, scale, ntau, nv, u[k]);
-    drop_masked(nv, g);
+    rectify(x, scale, ntau, valid_in_chunk(limit, c0), u[k]);
 #pragma unroll
     for (int j = 0; j < V; ++j) dy[k][j] = g[j];
     add_dot(u[k], lg[PMODE ? 0 : k], g);
   }
-  for (int64_t c0 = CH * SPAN + cl; c0 - cl < limit; c0 += SPAN) {
+  for (int64_t c0 = CH * SPAN + cl; MORE && c0 - cl < limit; c0 += SPAN) {
     if (c0 >= limit) continue;
     float x[V], g[V], uc[V], lc[V];
     load_chunk<T, ANY>(row, c0, a.N, x);
     load_chunk<T, ANY>(dyrow, c0, a.N, g);
-    const int nv = valid_in_chunk(limit, c0);
-    rectify(x, scale, ntau, nv, uc);
-    drop_masked(nv, g);
+    rectify(x, scale, ntau, valid_in_chunk(limit, c0), uc);
     add_dot(uc, lc, g);
   }
   dot = row_sum(dot);
-  if (PMODE) {
-    dot /= z;
-    // A power of the forward overflowed: its W held inf * 0, and no entry has a gradient (the
-    // unit's powers are finite, so the sum alone would end as 0).
-    if (pow_p<PMODE>(peak, a.p) == __builtin_inff()) dot = __builtin_nanf("");
-  }
+  if (PMODE) dot /= z;
+  if (dot != dot || (PMODE && z > __FLT_MAX__))
+    dot = plain_dot<T, PMODE>(a, row, dyrow, limit, lane, a.Z[r]);
 
   float gate = 1.0f, gterm = 0.0f;
   if (a.has_gamma) {
@@ -405,7 +412,7 @@ __global__ __launch_bounds__(256, CH == 1 ? 8 : CH == 2 ? (PMODE ? 6 : 5) : PMOD
     }
     if (c0 < a.N) store_chunk<T, ANY>(drow, c0, a.N, d);
   }
-  for (int64_t c0 = CH * SPAN + cl; c0 - cl < a.N; c0 += SPAN) {
+  for (int64_t c0 = CH * SPAN + cl; MORE && c0 - cl < a.N; c0 += SPAN) {
     if (c0 >= a.N) continue;
     float d[V] = {};
     if (c0 < limit) {
@@ -488,10 +495,10 @@ int launch_rows(const RowsArgs& a, hipStream_t st) {
   const int64_t ch = (a.N + 64 * V - 1) / (64 * V);
   if (vec && ch <= 1) launch_rows_v<T, false, 1, BWD>(a, pm, grid, block, st);
   else if (vec && ch == 2) launch_rows_v<T, false, 2, BWD>(a, pm, grid, block, st);
-  else if (vec) launch_rows_v<T, false, 4, BWD>(a, pm, grid, block, st);
+  else if (vec) launch_rows_v<T, false, kMaxChunks, BWD>(a, pm, grid, block, st);
   else if (ch <= 1) launch_rows_v<T, true, 1, BWD>(a, pm, grid, block, st);
   else if (ch == 2) launch_rows_v<T, true, 2, BWD>(a, pm, grid, block, st);
-  else launch_rows_v<T, true, 4, BWD>(a, pm, grid, block, st);
+  else launch_rows_v<T, true, kMaxChunks, BWD>(a, pm, grid, block, st);
   return launch_status(BWD ? "pnfx_pn_rows_bwd" : "pnfx_pn_rows_fwd");
 }
 
