@@ -1,7 +1,7 @@
 // Row-fused rectified power-norm score -> weight (the materialised-score path of pn_fir_tau).
 //
 // One wave64 per score row; any row length.  Forward makes two passes over the row:
-// pass 1 accumulates the row peak and the power mass (lane-local, then a wave butterfly),
+// pass 1 accumulates the row peak and the power mass (lane-local, then a wave reduction),
 // pass 2 counts peak ties and writes the weights from the register-held scores (re-reading
 // only what did not fit).  Backward mirrors it: pass 1 forms <dW, w_hat>, pass 2 writes
 // dScores and the row's tau partial.  A lane moves 16 bytes per access whatever the rows'
@@ -293,29 +293,13 @@ __device__ __forceinline__ float pow_pm1(float u) {
   }
 }
 
-// <dW, w_hat> of a row entry by entry over its valid columns, for rows where the backward's own sum
-// does not tell: it is NaN (a chunk's dW past the causal limit may be an infinity, times a power of 0),
-// or a power overflowed in the forward (inf / inf here; the backward's unit would end as 0).  A test
-// of each entry instead cost the backward 5-10 % (17.2 -> 18.1 us at [64, 1, 512, 512] bf16).
-template <typename T, int PMODE>
-__device__ __forceinline__ float plain_dot(const RowsArgs& a, const T* row, const T* dyrow,
-                                           int64_t limit, int lane, float z) {
-  const float ntau = -a.tau[0];
-  float dot = 0.0f;
-#pragma unroll 1
-  for (int64_t c = lane; c < limit; c += 64) {
-    const float u = fmaxf(__builtin_fmaf(to_f32(row[c]), a.scale, ntau), 0.0f);
-    dot = __builtin_fmaf(to_f32(dyrow[c]), pow_p<PMODE>(u, a.p) / z, dot);
-  }
-  return row_sum(dot);
-}
-
 // The backward takes the scores in units of the power of two of the row's peak for p = 10 and 2
 // (an exact scaling, folded into scale and tau): the powers are then at most 1, so that the sum
-// <dW, u^p> can be divided by Z once instead of entry by entry without overflowing.  Peaks below
-// 2^-16 keep that unit: their powers are below fp32's range in either.
+// <dW, u^p> can be divided by Z once instead of entry by entry without overflowing.  The unit is no
+// smaller than 2^-16: Z holds 1e-12, which for p = 10 is 2^120 in that unit's powers, and in a
+// smaller one would overflow.
 template <typename T, int PMODE, bool ANY, int CH>
-__global__ __launch_bounds__(256, CH == 1 ? 8 : CH == 2 ? (PMODE ? 6 : 5) : PMODE ? 4 : 3) void pn_rows_bwd_kernel(RowsArgs a) {
+__global__ __launch_bounds__(256, CH == 1 ? (PMODE ? 8 : 7) : CH == 2 ? (PMODE ? 6 : 5) : PMODE ? 4 : 3) void pn_rows_bwd_kernel(RowsArgs a) {
   constexpr int V = RowIO<T, ANY>::V;
   constexpr int64_t SPAN = 64 * V;
   constexpr bool MORE = CH == kMaxChunks;  // rows longer than the registers
@@ -376,8 +360,34 @@ __global__ __launch_bounds__(256, CH == 1 ? 8 : CH == 2 ? (PMODE ? 6 : 5) : PMOD
   }
   dot = row_sum(dot);
   if (PMODE) dot /= z;
-  if (dot != dot || (PMODE && z > __FLT_MAX__))
-    dot = plain_dot<T, PMODE>(a, row, dyrow, limit, lane, a.Z[r]);
+  // Rows whose sum does not tell: NaN may come from a chunk's dW past the causal limit (an infinity
+  // there, times a power of 0), and where a power overflowed in the forward (inf / inf) this unit's
+  // sum ends as 0.  The same sum over the valid entries alone.  (A test of each entry above instead
+  // cost 17.2 -> 18.1 us at [64, 1, 512, 512] bf16.)
+  if (dot != dot || (PMODE && z > __FLT_MAX__)) {
+    dot = 0.0f;
+    const auto add_valid = [&](int64_t c0, const float (&uc)[V], const float (&g)[V]) {
+      const int nv = valid_in_chunk(limit, c0);
+      float gv[V], lc[V];
+#pragma unroll
+      for (int j = 0; j < V; ++j) gv[j] = j < nv ? g[j] : 0.0f;
+      add_dot(uc, lc, gv);
+    };
+#pragma unroll
+    for (int k = 0; k < CH; ++k)
+      if (k * SPAN < limit) add_valid(k * SPAN + cl, u[k], dy[k]);
+    for (int64_t c0 = CH * SPAN + cl; MORE && c0 - cl < limit; c0 += SPAN) {
+      if (c0 >= limit) continue;
+      float x[V], g[V], uc[V];
+      load_chunk<T, ANY>(row, c0, a.N, x);
+      load_chunk<T, ANY>(dyrow, c0, a.N, g);
+      rectify(x, scale, ntau, valid_in_chunk(limit, c0), uc);
+      add_valid(c0, uc, g);
+    }
+    dot = row_sum(dot);
+    if (PMODE) dot /= z;
+    if (PMODE && pow_p<PMODE>(peak, a.p) > __FLT_MAX__) dot = __builtin_nanf("");
+  }
 
   float gate = 1.0f, gterm = 0.0f;
   if (a.has_gamma) {
