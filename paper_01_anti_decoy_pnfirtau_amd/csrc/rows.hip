@@ -6,7 +6,7 @@
 // only what did not fit).  Backward mirrors it: pass 1 forms <dW, w_hat>, pass 2 writes
 // dScores and the row's tau partial.  A lane moves 16 bytes per access whatever the rows'
 // alignment (rows that start at any element: unaligned vector accesses, and single elements
-// for a last chunk that the row does not fill).
+// for a last chunk that the row does not fill), but for short ragged bf16 rows (launch_rows).
 //
 // Bound: HBM for the bytes (the causal half of the inputs read, the whole output written), with
 // the vector units close behind: about 19 operations per entry forward and 27 backward.  On the
@@ -95,12 +95,17 @@ __device__ __forceinline__ float pow_p(float u, float p) {
   }
 }
 
-// A chunk of V consecutive elements of a row (16 bytes), converted to fp32.  ANY: rows of any
-// alignment and length, else rows of whole 16-byte aligned chunks.
-template <typename T, bool ANY>
+// A chunk of V consecutive elements of a row, converted to fp32: 16 bytes, or one element.  ANY: rows
+// of any alignment and length, else rows of whole 16-byte aligned chunks.
+template <typename T, int V, bool ANY>
 struct RowIO;
+template <typename T>
+struct RowIO<T, 1, true> {
+  __device__ static __forceinline__ void load(const T* p, float (&x)[1]) { x[0] = to_f32(*p); }
+  __device__ static __forceinline__ void store(T* p, const float (&x)[1]) { *p = from_f32<T>(x[0]); }
+};
 template <bool ANY>
-struct RowIO<bf16, ANY> {
+struct RowIO<bf16, 8, ANY> {
   static constexpr int V = 8;
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
   struct __attribute__((packed, aligned(ANY ? 2 : 16))) Raw { u32x4 q; };
@@ -121,7 +126,7 @@ struct RowIO<bf16, ANY> {
   }
 };
 template <bool ANY>
-struct RowIO<float, ANY> {
+struct RowIO<float, 4, ANY> {
   static constexpr int V = 4;
   struct __attribute__((packed, aligned(ANY ? 4 : 16))) Raw { f32x4 q; };
   __device__ static __forceinline__ void load(const float* p, float (&x)[V]) {
@@ -137,7 +142,7 @@ struct RowIO<float, ANY> {
 template <typename T, bool ANY, int V>
 __device__ __forceinline__ void load_chunk(const T* row, int64_t c0, int64_t N, float (&x)[V]) {
   if (!ANY || c0 + V <= N) {
-    RowIO<T, ANY>::load(row + c0, x);
+    RowIO<T, V, ANY>::load(row + c0, x);
   } else {
 #pragma unroll
     for (int j = 0; j < V; ++j) x[j] = c0 + j < N ? to_f32(row[c0 + j]) : 0.f;
@@ -146,7 +151,7 @@ __device__ __forceinline__ void load_chunk(const T* row, int64_t c0, int64_t N, 
 template <typename T, bool ANY, int V>
 __device__ __forceinline__ void store_chunk(T* row, int64_t c0, int64_t N, const float (&x)[V]) {
   if (!ANY || c0 + V <= N) {
-    RowIO<T, ANY>::store(row + c0, x);
+    RowIO<T, V, ANY>::store(row + c0, x);
   } else {
 #pragma unroll
     for (int j = 0; j < V; ++j)
@@ -181,9 +186,8 @@ constexpr int kMaxChunks = 4;
 // power, whose exponential and logarithm make most of the kernel, is kept in registers, in the
 // backward its logarithm ([64, 1, 512, 512] bf16 at p = 3.5: forward 30.8 -> 21.5 us, backward 36.4 ->
 // 33.4).
-template <typename T, int PMODE, bool ANY, int CH>
-__global__ __launch_bounds__(256, CH <= 2 ? 8 : 4) void pn_rows_fwd_kernel(RowsArgs a) {
-  constexpr int V = RowIO<T, ANY>::V;
+template <typename T, int PMODE, int V, bool ANY, int CH>
+__global__ __launch_bounds__(256, V == 1 || CH <= 2 ? 8 : 4) void pn_rows_fwd_kernel(RowsArgs a) {
   constexpr int64_t SPAN = 64 * V;
   constexpr bool MORE = CH == kMaxChunks;  // rows longer than the registers
   const int64_t r = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -298,9 +302,8 @@ __device__ __forceinline__ float pow_pm1(float u) {
 // <dW, u^p> can be divided by Z once instead of entry by entry without overflowing.  The unit is no
 // smaller than 2^-16: Z holds 1e-12, which for p = 10 is 2^120 in that unit's powers, and in a
 // smaller one would overflow.
-template <typename T, int PMODE, bool ANY, int CH>
-__global__ __launch_bounds__(256, CH == 1 ? (PMODE ? 8 : 7) : CH == 2 ? (PMODE ? 6 : 5) : PMODE ? 4 : 3) void pn_rows_bwd_kernel(RowsArgs a) {
-  constexpr int V = RowIO<T, ANY>::V;
+template <typename T, int PMODE, int V, bool ANY, int CH>
+__global__ __launch_bounds__(256, V == 1 ? 8 : CH == 1 ? (PMODE ? 8 : 7) : CH == 2 ? (PMODE ? 6 : 5) : PMODE ? 4 : 3) void pn_rows_bwd_kernel(RowsArgs a) {
   constexpr int64_t SPAN = 64 * V;
   constexpr bool MORE = CH == kMaxChunks;  // rows longer than the registers
   const int64_t r = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -477,21 +480,27 @@ __global__ __launch_bounds__(1024) void sum_f64_kernel(const S* x, int64_t n, do
   }
 }
 
-template <typename T, bool ANY, int CH, bool BWD>
+template <typename T, int V, bool ANY, int CH, bool BWD>
 void launch_rows_v(const RowsArgs& a, int pm, dim3 grid, dim3 block, hipStream_t st) {
   if (BWD) {
-    if (pm == 10) hipLaunchKernelGGL((pn_rows_bwd_kernel<T, 10, ANY, CH>), grid, block, 0, st, a);
-    else if (pm == 2) hipLaunchKernelGGL((pn_rows_bwd_kernel<T, 2, ANY, CH>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((pn_rows_bwd_kernel<T, 0, ANY, CH>), grid, block, 0, st, a);
+    if (pm == 10) hipLaunchKernelGGL((pn_rows_bwd_kernel<T, 10, V, ANY, CH>), grid, block, 0, st, a);
+    else if (pm == 2) hipLaunchKernelGGL((pn_rows_bwd_kernel<T, 2, V, ANY, CH>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((pn_rows_bwd_kernel<T, 0, V, ANY, CH>), grid, block, 0, st, a);
   } else {
-    if (pm == 10) hipLaunchKernelGGL((pn_rows_fwd_kernel<T, 10, ANY, CH>), grid, block, 0, st, a);
-    else if (pm == 2) hipLaunchKernelGGL((pn_rows_fwd_kernel<T, 2, ANY, CH>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((pn_rows_fwd_kernel<T, 0, ANY, CH>), grid, block, 0, st, a);
+    if (pm == 10) hipLaunchKernelGGL((pn_rows_fwd_kernel<T, 10, V, ANY, CH>), grid, block, 0, st, a);
+    else if (pm == 2) hipLaunchKernelGGL((pn_rows_fwd_kernel<T, 2, V, ANY, CH>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((pn_rows_fwd_kernel<T, 0, V, ANY, CH>), grid, block, 0, st, a);
   }
 }
 
 // Rows of one or two chunks (64 lanes x 16 bytes) hold them in registers, longer ones up to four
 // (fewer registers, more waves: two for four at N = 777 bf16 took the backward from 28 to 23.3 us).
+// Short bf16 rows that are not whole aligned chunks go by single elements, 64 to a register: with
+// eight to a lane few lanes compute, and the row's part of a chunk takes eight branches.  Forward /
+// backward over 2^24 scores, by chunks -> by elements: N = 33 160 / 220 -> 89 / 137 us, N = 129
+// 44.3 / 60.5 -> 35.1 / 52.5, N = 190 31.9 / 44.8 -> 26.6 / 38.9, N = 257 24.1 / 32.8 -> 25.8 / 37.5; with
+// the general power, which is mostly computing, N = 300 34.5 / 57 -> 26.9 / 37.2, N = 511 22.5 /
+// 36.4 -> 23.5 / 34.3.
 template <typename T, bool BWD>
 int launch_rows(const RowsArgs& a, hipStream_t st) {
   const dim3 grid((unsigned)((a.R + 3) / 4)), block(256);
@@ -503,12 +512,20 @@ int launch_rows(const RowsArgs& a, hipStream_t st) {
   const bool vec = a.N % V == 0 && aligned(a.raw, a.raw_rs) && aligned(a.out, a.out_rs) &&
                    (!BWD || aligned(a.dw, a.dw_rs));
   const int64_t ch = (a.N + 64 * V - 1) / (64 * V);
-  if (vec && ch <= 1) launch_rows_v<T, false, 1, BWD>(a, pm, grid, block, st);
-  else if (vec && ch == 2) launch_rows_v<T, false, 2, BWD>(a, pm, grid, block, st);
-  else if (vec) launch_rows_v<T, false, kMaxChunks, BWD>(a, pm, grid, block, st);
-  else if (ch <= 1) launch_rows_v<T, true, 1, BWD>(a, pm, grid, block, st);
-  else if (ch == 2) launch_rows_v<T, true, 2, BWD>(a, pm, grid, block, st);
-  else launch_rows_v<T, true, kMaxChunks, BWD>(a, pm, grid, block, st);
+  if constexpr (sizeof(T) == 2) {
+    if (!vec && a.N <= (pm ? 256 : 384)) {
+      if (a.N <= 64) launch_rows_v<T, 1, true, 1, BWD>(a, pm, grid, block, st);
+      else if (a.N <= 128) launch_rows_v<T, 1, true, 2, BWD>(a, pm, grid, block, st);
+      else launch_rows_v<T, 1, true, 6, BWD>(a, pm, grid, block, st);
+      return launch_status(BWD ? "pnfx_pn_rows_bwd" : "pnfx_pn_rows_fwd");
+    }
+  }
+  if (vec && ch <= 1) launch_rows_v<T, V, false, 1, BWD>(a, pm, grid, block, st);
+  else if (vec && ch == 2) launch_rows_v<T, V, false, 2, BWD>(a, pm, grid, block, st);
+  else if (vec) launch_rows_v<T, V, false, kMaxChunks, BWD>(a, pm, grid, block, st);
+  else if (ch <= 1) launch_rows_v<T, V, true, 1, BWD>(a, pm, grid, block, st);
+  else if (ch == 2) launch_rows_v<T, V, true, 2, BWD>(a, pm, grid, block, st);
+  else launch_rows_v<T, V, true, kMaxChunks, BWD>(a, pm, grid, block, st);
   return launch_status(BWD ? "pnfx_pn_rows_bwd" : "pnfx_pn_rows_fwd");
 }
 

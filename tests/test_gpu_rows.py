@@ -77,10 +77,10 @@ def test_rows_of_length_one_and_many_rows(dev):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("p", [10.0, 2.0, 3.5])
-@pytest.mark.parametrize("N", [1, 7, 9, 255, 257, 511, 513, 1023, 1025, 2051])
+@pytest.mark.parametrize("N", [1, 7, 9, 63, 65, 127, 129, 255, 257, 383, 385, 511, 513, 1023, 1025, 2051])
 def test_rows_ends_of_chunks_match_oracle(dev, dtype, N, p):
     """Rows that start at any element and end within a 16-byte chunk, one to five register chunks
-    long, forward and backward."""
+    long, forward and backward; short bf16 rows that go by elements, one to six registers long."""
     print(f"[rows N={N} p={p} {dtype}]", flush=True)
     from paper_01_anti_decoy_pnfirtau_amd.hip_pnfirtau import hip_pn_fir_tau_scores
     raw = seeded((1, 1, N, N), 30, dtype, dev, scale=2.0).requires_grad_()
