@@ -53,6 +53,20 @@ struct QBuf {
   float* rc;  // [planes][64 rows]
 };
 
+// The columns past d of a ragged head's key tile are zero for the scores: Q is zero there, but against
+// an infinity that the tile re-loads the score would be NaN, which the rectifier drops.  Up to 96
+// columns the tile's loads leave them out (forward at B=2 H=8 N=4096 d=40 92 -> 95 us, d=80 none); at 128
+// the masks of those loads do not fit the registers (d=104 123 -> 140), and the last k-step's fragment,
+// whose lane groups past d are whole, is masked instead (123 -> 126).
+constexpr bool key_and_mask(int D) { return D == 128; }
+__device__ __forceinline__ bf16x8 and_frag(bf16x8 v, uint32_t m) {
+  return __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, v) & u32x4{m, m, m, m});
+}
+template <int D>
+__device__ __forceinline__ uint32_t frag_mask(int g, int d) {
+  return 8 * (4 * (k_steps(D) - 1) + g) < d ? ~0u : 0u;
+}
+
 // Multiply the 8 bf16 values of a fragment by an exact power of two (no rounding).
 __device__ __forceinline__ bf16x8 scale_frag(bf16x8 v, float s) {
 #pragma unroll
@@ -295,6 +309,7 @@ __global__ __launch_bounds__(256, D <= 64 && !FIRK ? 3 : 2) void flash_fwd_kerne
   const float ntau = -p.tau[0];
   const float scale = p.scale;
   const FragLane flr = rt_lane<DK>(r16, g), flt = tr_lane<DK>(lane);
+  const uint32_t kmask = frag_mask<D>(g, d);
 
   // The silent-tile bound applies (key norms given, tau > 0: at tau <= 0 no tile but an
   // all-zero one can be bounded silent, and the kernel then runs without it).
@@ -404,7 +419,12 @@ __global__ __launch_bounds__(256, D <= 64 && !FIRK ? 3 : 2) void flash_fwd_kerne
 
   // Software pipeline: tile t+1 streams from HBM/L2 straight into one LDS buffer while tile
   // t is computed from the other; one barrier per tile.
-  const TileDma<D, DK> kdma(w, lane, p.ksn, d), vdma(w, lane, p.vsn, d);
+  const TileDma<D, DK, RAG && !key_and_mask(D)> kdma(w, lane, p.ksn, d);
+  const TileDma<D, DK> vdma(w, lane, p.vsn, d);
+  if (RAG && !key_and_mask(D)) {
+    kdma.clear_tail(Ks0, w, lane);
+    kdma.clear_tail(Ks1, w, lane);
+  }
   auto load_tile = [&](int n, const KVBuf& bb) {
     if constexpr (FIRK) {
       // raw rows n - 8 .. n + 63, KCPR chunks each (72 KCPR chunks, 64 per wave and load);
@@ -511,6 +531,7 @@ __global__ __launch_bounds__(256, D <= 64 && !FIRK ? 3 : 2) void flash_fwd_kerne
           bf16x8 kf[KS];
 #pragma unroll
           for (int ks = 0; ks < KS; ++ks) kf[ks] = ld16(Kc + rt_frag<DK>(flr, 2 * hf + kk, ks));
+          if (RAG && key_and_mask(D)) kf[KS - 1] = and_frag(kf[KS - 1], kmask);
 #pragma unroll
           for (int qb = 0; qb < 2; ++qb) {
             f32x4 a4 = s_init;
@@ -809,6 +830,7 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dq_kernel(BwdParams p) {
   // reference rounds it; at scale = 0 (dS = 0), f = 1 keeps du for the tau partials.
   const float fdu = scale != 0.f ? scale : 1.f;
   const FragLane flr = rt_lane<DK>(r16, g), flt = tr_lane<DK>(lane);
+  const uint32_t kmask = frag_mask<D>(g, d);
 
   bf16x8 qf[QB][KS], dof[QB][KS];
   // Row constants.  The scores of row i are formed scaled by 2^-e_i, e_i the exponent of its
@@ -915,7 +937,12 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dq_kernel(BwdParams p) {
     return ident ? e : __builtin_amdgcn_readfirstlane((int)tl_s[min(e, nlist - 1)]);
   };
 
-  const TileDma<D, DK> kdma(w, lane, p.ksn, d), vdma(w, lane, p.vsn, d);
+  const TileDma<D, DK, RAG && !key_and_mask(D)> kdma(w, lane, p.ksn, d);
+  const TileDma<D, DK> vdma(w, lane, p.vsn, d);
+  if (RAG && !key_and_mask(D)) {
+    kdma.clear_tail(Ks0, w, lane);
+    kdma.clear_tail(Ks1, w, lane);
+  }
   auto load_tile = [&](int n, const KVBuf& bb) {
     kdma.load(K, p.ksn, n, N, bb.k, w, d - 8);
     vdma.load(V, p.vsn, n, N, bb.v, w, d - 8);
@@ -956,6 +983,7 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_dq_kernel(BwdParams p) {
             kf[ks] = ld16(Kc + off);
             vf[ks] = ld16(Vc + off);
           }
+          if (RAG && key_and_mask(D)) kf[KS - 1] = and_frag(kf[KS - 1], kmask);
 #pragma unroll
           for (int qb = 0; qb < QB; ++qb) {
             f32x4 a4 = s_init[qb], c4 = dw_init[qb];
@@ -1537,7 +1565,7 @@ int launch_bwd_d(const BwdParams& bp_in, bool causal, bool has_gamma, int stages
 
 // Rows of fewer columns than the kernel's head size: the same kernels with the range tests of RAG, no
 // scale folded in (PS) whatever it is, so that the backward recomputes the forward's scores.  The
-// tests lie in the prologue and epilogue; the loop is that of the full rows.  Padded copies of the
+// tests lie in the prologue, the epilogue and the key tiles (key_and_mask).  Padded copies of the
 // operands instead (and slices of the results) took 110 of 229 us at B=4 H=8 N=1000 d=80, where
 // this takes 103 us in all; 96 columns rather than 128 save a quarter of the products.
 template <int D>

@@ -118,12 +118,14 @@ __device__ __forceinline__ void lds_dma16(const bf16* src, bf16* dst) {
 __device__ __forceinline__ int row_of_slot(int s) {  // inverse of slot_of
   return (s & 32) | ((s & 12) << 1) | ((s >> 2) & 4) | (s & 3);
 }
-// `d` <= D: the columns that the rows hold; chunks past them re-load the row's last one.
-template <int D, int DK>
+// `d` <= D: the columns that the rows hold; chunks past them re-load the row's last one.  ZERO: they are
+// left alone instead, and clear_tail makes them 0 once.
+template <int D, int DK, bool ZERO = false>
 struct TileDma {
   static constexpr int CPR = DK / 8;      // 16-byte chunks per tile row
   static constexpr int NI = 64 * CPR / 256;  // loads per thread
   static constexpr bool PART = D > 32 && D < DK;  // chunks past D are left alone
+  static constexpr bool SKIP = PART || ZERO;      // some chunks (col D here) are
   int row[NI], col[NI];
   unsigned off[NI];  // byte offset of the lane's chunks from the tile's first row
   __device__ __forceinline__ TileDma(int w, int lane, int64_t sn, int d = D) {
@@ -133,9 +135,16 @@ struct TileDma {
       const int slot = L / CPR, pos = L % CPR;
       const int ch = pos ^ swz_rt<DK>(slot);
       row[j] = row_of_slot(slot);
-      col[j] = d == D ? 8 * (PART ? ch : ch % (D / 8)) : min(8 * ch, PART && ch >= D / 8 ? D : d - 8);
+      if (ZERO) col[j] = 8 * ch < d ? 8 * ch : D;
+      else col[j] = d == D ? 8 * (PART ? ch : ch % (D / 8)) : min(8 * ch, PART && ch >= D / 8 ? D : d - 8);
       off[j] = (unsigned)(2 * (row[j] * sn + col[j]));
     }
+  }
+  // Before the first load into `tile`; published with it.
+  __device__ __forceinline__ void clear_tail(bf16* tile, int w, int lane) const {
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+      if (col[j] >= D) *reinterpret_cast<bf16x8*>(tile + (4 * j + w) * 512 + 8 * lane) = zero_bf16x8();
   }
   // A whole tile (row0 + 64 <= N) is a wave-uniform base plus 32-bit lane offsets, which the
   // load takes as scalar base + vector offset: no per-load address arithmetic.
@@ -145,7 +154,7 @@ struct TileDma {
       const char* base = reinterpret_cast<const char*>(src + (int64_t)row0 * sn);
 #pragma unroll
       for (int j = 0; j < NI; ++j)
-        if (!PART || col[j] < D)
+        if (!SKIP || col[j] < D)
           lds_dma16(reinterpret_cast<const bf16*>(base + off[j]), tile + (4 * j + w) * 512);
     } else {
       load_clamped(src, sn, row0, N, tile, w, d_last);
@@ -158,7 +167,7 @@ struct TileDma {
 #pragma unroll
     for (int j = 0; j < NI; ++j) {
       const int r = min(row0 + row[j], N - 1);
-      if (!PART || col[j] < D)
+      if (!SKIP || col[j] < D)
         lds_dma16(src + (int64_t)r * sn + min(col[j], d_last), tile + (4 * j + w) * 512);
     }
   }

@@ -130,3 +130,29 @@ def test_flash_ragged_head_is_the_padded_head(dev, d, N, causal, packed):
     for name, a, b in zip(("O", "dq", "dk", "dv"), got, want):
         assert torch.equal(a, b[..., :d]), name
     assert torch.equal(got[4], want[4])
+
+
+@pytest.mark.parametrize("d", [8, 24, 40, 72, 80, 120])
+def test_flash_ragged_head_infinite_key_stays_visible(dev, d):
+    """An infinite key entry in the last columns of a ragged head: O and dq are finite exactly where
+    those of the zero-padded rows with one kernel size more are (a query that scores +inf against the
+    key is not, and the key is not dropped)."""
+    print(f"[flash ragged inf d={d}]", flush=True)
+    B, H, N = 1, 2, 150
+    full = 32 if d < 32 else 64 if d < 64 else 128
+    q, k, v, dO = (seeded((B, H, N, d), 550 + i, torch.bfloat16, dev) for i in range(4))
+    k[0, 0, 37, d - 1] = float("inf")
+
+    def run(*ts):
+        t0 = torch.tensor(0.0, device=dev)
+        leaves = [t.detach().requires_grad_() for t in ts[:3]]
+        o = flash_pn_fir_tau_attention(*leaves, t0, scale=0.3)
+        return o.detach(), torch.autograd.grad(o, leaves[0], ts[3])[0]
+
+    got = run(q, k, v, dO)
+    want = run(*(torch.nn.functional.pad(t, (0, full - d)) for t in (q, k, v, dO)))
+    for a, b in zip(got, want):
+        assert torch.equal(torch.isfinite(a), torch.isfinite(b[..., :d]))
+    hit = (q[0, 0, :, d - 1] > 0) & (torch.arange(N, device=dev) >= 37)
+    assert torch.equal(torch.isfinite(got[0]).all(-1)[0, 0], ~hit) and hit.any()
+    assert torch.isfinite(got[0][0, 1]).all()
