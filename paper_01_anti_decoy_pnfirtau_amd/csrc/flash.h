@@ -51,15 +51,23 @@ struct BwdParams {
   int d = 0;    // bf16: columns of a row of the operands (at most the kernel's head size)
 };
 
-// (b, h) slices per dispatch group of the bf16 kernels: as many as keep the group's streamed pair of
-// operands (N rows of 4 D bytes a slice) within one XCD's 4 MiB of L2, at least two.  Larger groups
-// dispatch more heavy causal blocks first, so fewer run alone at the end; groups past the L2 re-read
-// their tiles from beyond it (at B=4 H=16 N=8192 d=64, two slices, groups of four took 2-3x the
-// misses for nothing in the gradients).  With half the key tiles silent at B=4 H=16 N=4096 d=64, groups
-// of four instead of two: dK/dV 258 -> 213 us, forward 130 -> 125.
-inline int slice_group(int64_t N, int64_t D) {
-  const int64_t g = (4ll << 20) / (N * D * 4);
-  return (int)(g < 2 ? 2 : g > 64 ? 64 : g);
+// (b, h) slices per dispatch group of the bf16 kernels: the eighth of BH slices that an XCD owns in
+// groups of one size, about as many as keep the group's streamed pair of operands (N rows of 4 D bytes
+// a slice) within one XCD's 4 MiB of L2, at least two.  Larger groups dispatch more heavy causal blocks
+// first, so fewer run alone at the end; groups past the L2 re-read their tiles from beyond it (at
+// B=4 H=16 N=8192 d=64, two slices, groups of four took 2-3x the misses for nothing in the gradients).
+// With half the key tiles silent at B=4 H=16 N=4096 d=64, groups of four instead of two: dK/dV 258 ->
+// 213 us, forward 130 -> 125.  A last group smaller than the others starts its heavy blocks late, on a
+// chip that it does not fill: six slices (BH=48 N=3000 d=64) as five and one took 118 us forward and
+// 362 backward, as one group of six 89 and 274 (in pairs 93 and 326); eight (BH=64 N=1100 d=128) as
+// seven and one 50 and 176, as one group 41 and 138 (45 and 157).
+inline int slice_group(int64_t N, int64_t D, int64_t BH) {
+  int64_t g = (4ll << 20) / (N * D * 4);
+  g = g < 2 ? 2 : g > 64 ? 64 : g;
+  const int64_t own = BH / 8;
+  if (own <= g) return (int)g;
+  const int64_t groups = (2 * own + g) / (2 * g);  // own / g, rounded
+  return (int)((own + groups - 1) / groups);
 }
 
 // Head size of the kernel that takes rows of D columns: D itself for the sizes with a kernel of their

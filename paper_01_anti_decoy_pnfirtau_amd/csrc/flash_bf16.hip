@@ -92,26 +92,35 @@ __device__ __forceinline__ float pow10f_(float u) {
 // Map a linear block id to (bh, block index).  Each XCD (block id % 8 on the round-robin
 // dispatcher) owns BH / 8 whole (b, h) slices, so their K/V (forward, dQ) or Q/dO (dK/dV) tiles
 // stay in that XCD's L2; the blocks of the BH % 8 slices left over are dealt to all XCDs in turn,
-// mixed evenly among the owned ones.  Own slices go in groups of `grp`, and a group's blocks are
-// dispatched heaviest first across its slices: causal blocks range from one tile of work to N/64,
-// and in smaller groups the last group's heavy blocks start late and run alone.  See slice_group
-// for the size of the groups.
+// mixed evenly among the owned ones, the first dealt one first (last, a slice's longest blocks shared
+// a CU with the owned ones': BH=33 N=1100 d=64 forward 31.2 us, 28.2 so).  Own slices go in groups of
+// `grp`, and a group's blocks are dispatched heaviest first across its slices: causal blocks range
+// from one tile of work to N/64, and in smaller groups the last group's heavy blocks start late and run
+// alone.  See slice_group for the size of the groups.
+constexpr unsigned kCUs = 256;
 __device__ __forceinline__ void map_block(int nblk, int BH, int grp, bool heavy_last_index, int& bh,
                                           int& blk) {
   const unsigned xcd = blockIdx.x & 7, own = (unsigned)BH >> 3, left = (unsigned)BH & 7;
   unsigned r = blockIdx.x >> 3;  // the XCD's r-th workgroup
   unsigned first = xcd * own, ge = own;
   bool dealt = false;
-  if (left) {
-    // The XCD's sequence mixes its n_own own blocks with the n_left dealt to it: p0 own ones come
-    // before its i-th workgroup.
+  if (left && (unsigned)(nblk * BH) <= kCUs) {  // a CU for every block: no order, all are dealt
+    dealt = true;
+    r = blockIdx.x;
+    first = 0;
+    ge = BH;
+  } else if (left) {
+    // The XCD's sequence mixes its n_own own blocks with the n_left dealt to it, a dealt one ahead of
+    // every BH / left - 1 own ones: q0 dealt ones come before its i-th workgroup, q1 before the next.
     const unsigned i = r, n_own = own * nblk, n_left = (left * nblk - xcd + 7) >> 3;
-    const auto own_before = [&](unsigned k) {
-      const unsigned m = min(k - k * left / (unsigned)BH, n_own);
+    const unsigned num = i * left + (unsigned)BH - 1, q0 = num / (unsigned)BH;
+    const unsigned q1 = q0 + (num - q0 * (unsigned)BH + left >= (unsigned)BH);
+    const auto own_before = [&](unsigned k, unsigned q) {
+      const unsigned m = min(k - min(q, k), n_own);
       return k > n_left ? max(m, k - n_left) : m;
     };
-    r = own_before(i);
-    if (own_before(i + 1) == r) {
+    r = own_before(i, q0);
+    if (own_before(i + 1, q1) == r) {
       dealt = true;
       r = (i - r) * 8 + xcd;  // index among all the dealt blocks
       first = 8 * own;

@@ -123,7 +123,7 @@ static int flash_fwd_impl(bool any, const void* q, int64_t qsb, int64_t qsh, int
   FwdParams fp{q, k, v, o, o_lo, qsb, qsh, qsn, ksb, ksh, ksn, vsb, vsh, vsn, osb, osh, osn,
                M, Z, Nmax, tile_mask, static_cast<float*>(workspace), (int)B, (int)H, (int)N,
                (int)((N + 31) / 32), (int)((N + 63) / 64), tau, scale, gamma, has_gamma != 0};
-  fp.grp = slice_group(N, D);
+  fp.grp = slice_group(N, D, B * H);
   fp.d = (int)D;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (!own_kernel_dim(D)) return flash_fwd_ragged_bf16(fp, causal != 0, st);
@@ -179,7 +179,7 @@ extern "C" int pnfx_flash_fwd_fir(const void* q, int64_t qsb, int64_t qsh, int64
   FwdParams fp{q, k_raw, v, o, o_lo, qsb, qsh, qsn, ksb, ksh, ksn, vsb, vsh, vsn, osb, osh, osn,
                M, Z, nullptr, tile_mask, nullptr, (int)B, (int)H, (int)N,
                (int)((N + 31) / 32), (int)((N + 63) / 64), tau, scale, gamma, has_gamma != 0,
-               taps, (int)taps_rows, K, slice_group(N, D), (int)D};
+               taps, (int)taps_rows, K, slice_group(N, D, B * H), (int)D};
   return flash_fwd_fir_bf16(fp, D, causal != 0, reinterpret_cast<hipStream_t>(stream));
 }
 
@@ -235,7 +235,7 @@ static int flash_bwd_impl(bool any, int stages, const void* q, int64_t qsb, int6
                dqsb, dqsh, dqsn, dksb, dksh, dksn, dvsb, dvsh, dvsn,
                M, Z, tile_mask, rcbuf, parts, qs, ktact, amap, dtau,
                (int)B, (int)H, (int)N, (int)((N + 31) / 32), (int)((N + 63) / 64),
-               bwd_nkvb(N, D), tau, scale, gamma, slice_group(N, D), (int)D};
+               bwd_nkvb(N, D), tau, scale, gamma, slice_group(N, D, B * H), (int)D};
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (!own_kernel_dim(D)) return flash_bwd_ragged_bf16(bp, causal != 0, has_gamma != 0, st);
   return dtype == PNFX_BF16 ? flash_bwd_bf16(bp, D, causal != 0, has_gamma != 0, stages, st)

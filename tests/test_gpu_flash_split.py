@@ -21,8 +21,11 @@ def _grads(q, k, v, tau_val, dO, causal=True):
 
 @pytest.mark.parametrize("B,H,N,D", [
     (1, 1, 300, 64), (1, 6, 300, 64), (2, 4, 257, 16), (1, 11, 300, 32), (4, 5, 130, 128),
-    (67, 1, 2100, 64),   # eight whole slices per XCD in groups of seven, and three dealt out
+    (67, 1, 2100, 64),   # eight whole slices per XCD in one group, and three dealt out
     (9, 3, 4100, 128),   # three per XCD in groups of two
+    (33, 1, 1100, 64),   # one dealt out, ahead of the owned ones
+    (6, 8, 3000, 64),    # six per XCD in one group
+    (19, 8, 1100, 128),  # nineteen per XCD in three groups of seven, seven and five
 ])
 def test_flash_slices_do_not_depend_on_the_grid(dev, B, H, N, D):
     """Every slice of a call is bitwise the slice computed alone: each (slice, block) pair is
