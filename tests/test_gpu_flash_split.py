@@ -59,15 +59,30 @@ def test_flash_f32_edges_of_tiles_match_oracle(dev, N, D, aligned, causal):
 
 
 def test_flash_f32_last_value_row_not_finite(dev):
-    """An infinite last row of V reaches the last query alone: the rows that pad the last tile do
-    not carry it to the others."""
+    """An infinite last row of V makes the last query's output infinite, not NaN, which the rows that
+    pad the last tile by repeating it would (their weight 0 times an infinity), and reaches no query
+    of another 16-key block.  (Queries that share the last row's block, 64 .. 68 here, hold its masked
+    weight 0 times an infinity: NaN, as a dense product would.)"""
     N, D = 70, 64
     q, k, v, _ = (seeded((1, 1, N, D), 520 + i, torch.float32, dev) for i in range(4))
     k[..., -1, :] = q[..., -1, :]  # the last query attends to the last key
     v[..., -1, :] = float("inf")
     o = flash_pn_fir_tau_attention(q, k, v, torch.tensor(0.0, device=dev))
     assert torch.isfinite(o[..., :64, :]).all()
-    assert not torch.isfinite(o[..., -1, :]).any()
+    assert torch.isinf(o[..., -1, :]).all()
+
+
+@pytest.mark.parametrize("N", [70, 133])
+def test_flash_f32_last_gradient_row_not_finite(dev, N):
+    """An infinite last row of dO makes the dV of every key that the last query attends to infinite,
+    not NaN: the rows that pad the last query tile by repeating it add nothing."""
+    D = 64
+    q, k, v, dO = (seeded((1, 1, N, D), 525 + i, torch.float32, dev).abs() for i in range(4))
+    dO[..., -1, :] = float("inf")
+    leaves = [t.requires_grad_() for t in (q, k, v)]
+    o = flash_pn_fir_tau_attention(*leaves, torch.tensor(0.0, device=dev))
+    dv = torch.autograd.grad(o, v, dO)[0]
+    assert torch.isinf(dv).all()
 
 
 def test_flash_f32_backward_stages_called_separately(dev):
@@ -133,6 +148,36 @@ def test_flash_ragged_head_is_the_padded_head(dev, d, N, causal, packed):
     for name, a, b in zip(("O", "dq", "dk", "dv"), got, want):
         assert torch.equal(a, b[..., :d]), name
     assert torch.equal(got[4], want[4])
+
+
+@pytest.mark.parametrize("d", [8, 24, 40, 56, 80, 104])
+def test_flash_ragged_head_skips_silent_keys(dev, d):
+    """Blocks of zero keys under tau > 0, at a size where the forward takes the silent-tile bound (key
+    norms over the d columns that exist, heads up to 64): bitwise the zero-padded rows, tile mask
+    included, and the bound does skip (no positive score in those blocks)."""
+    print(f"[flash ragged silent d={d}]", flush=True)
+    B, H, N = 4, 4, 2080
+    full = 16 if d < 16 else 32 if d < 32 else 64 if d < 64 else 128
+    q, k, v, dO = (seeded((B, H, N, d), 560 + i, torch.bfloat16, dev) for i in range(4))
+    for j in range(0, N, 128):
+        k[:, :, j:j + 64] = 0
+    tau, scale = torch.tensor(0.25, device=dev), 0.3
+    assert B * H * N * N >= 1 << 26  # the op takes the bound from here on
+
+    def run(*ts):
+        o, o_lo, M, Z, _, mask = torch.ops.pnfx.flash_fwd(*ts[:3], tau, scale, 0.5, True, True, False,
+                                                          False)
+        grads = torch.ops.pnfx.flash_bwd(*ts[:3], tau, o, o_lo, ts[3], M, Z, mask, scale, 0.5, True,
+                                         True)
+        return [o, *grads[:3]], [M, Z, mask, grads[3]]
+
+    (got, gs), (want, ws) = run(q, k, v, dO), run(*(torch.nn.functional.pad(t, (0, full - d))
+                                                    for t in (q, k, v, dO)))
+    for a, b in zip(got, want):
+        assert torch.equal(a, b[..., :d])
+    for a, b in zip(gs, ws):
+        assert torch.equal(a, b)
+    assert not gs[2][:, :, 0::2].any() and gs[2][:, -1, 1:-1:2].all()
 
 
 @pytest.mark.parametrize("d", [8, 24, 40, 72, 80, 120])

@@ -52,6 +52,32 @@ def test_opcheck_fir_and_row_scores(dev, dtype):
                            True, True))
 
 
+@pytest.mark.parametrize("wide", [True, False])
+def test_opcheck_sum_and_linear(dev, wide):
+    torch.library.opcheck(torch.ops.pnfx.sum_f64.default, (seeded((700,), 322, device=dev), wide))
+    x = seeded((2, 40, 24), 323, torch.bfloat16, dev).requires_grad_(True)
+    w = seeded((16, 24), 324, torch.float32 if wide else torch.bfloat16, dev).requires_grad_(True)
+    # (the gradients' check runs the library's product where autograd records the backward)
+    torch.library.opcheck(torch.ops.pnfx.linear.default, (x, w))
+    dy = seeded((80, 16), 325, torch.bfloat16, dev)
+    torch.library.opcheck(torch.ops.pnfx.linear_wgrad.default,
+                          (dy, x.detach().reshape(80, 24), wide))
+
+
+@pytest.mark.parametrize("causal", [True, False])
+def test_opcheck_attention_on_projection_rows(dev, causal):
+    B, N, H, d = 2, 70, 3, 24
+    qkv = seeded((B, N, 3 * H * d), 326, torch.bfloat16, dev).requires_grad_(True)
+    taps, tau = torch.rand(7, device=dev), torch.tensor(0.05, device=dev, requires_grad=True)
+    args = (d ** -0.5, 0.5, True, causal)
+    torch.library.opcheck(torch.ops.pnfx.attn_rows.default, (qkv, taps, tau, H, *args))
+    qkv, tau = qkv.detach(), tau.detach()
+    o, o_lo, k, M, Z, mask = torch.ops.pnfx.attn_rows(qkv, taps, tau, H, *args)
+    dO = seeded((B, N, H * d), 327, torch.bfloat16, dev)
+    torch.library.opcheck(torch.ops.pnfx.attn_rows_bwd.default,
+                          (qkv, k, taps, tau, o, o_lo, dO, M, Z, mask, *args))
+
+
 def test_tau_on_the_host_is_moved_to_the_device(dev):
     """The kernels read tau on the device: a CPU (or bf16) tau tensor is brought to the
     operands' device as fp32 by the op, and its gradient comes back on tau's own device."""
