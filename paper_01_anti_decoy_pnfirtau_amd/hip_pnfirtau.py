@@ -89,16 +89,19 @@ def hip_pn_fir_tau_scores(
 PLAIN = (torch.Tensor, torch.nn.Parameter)  # neither a subclass nor a stand-in without memory
 
 
-def split_wgrad_applies(rows: int, out_features: int, in_features: int) -> bool:
+def split_wgrad_applies(rows: int, out_features: int, in_features: int, wide: bool = True) -> bool:
     """Whether pnfx::linear_wgrad is the faster weight gradient: many rows over a small weight, where
     one workgroup per output tile leaves the chip idle.  Measured on MI355X (us, this kernel against
     the library product and its cast to fp32): 768x256 over 16384 rows 29 / 93, over 2048 12 / 17,
     over 512 9.8 / 10.0; 1536x512 over 8192 42 / 55, over 2048 24 / 19; 768x768 over 8192 36 / 51,
     over 2048 22 / 18; 1024x1024 over 8192 34 / 56; 2304x768 over 16384 127 / 124; 3072x1024 over
-    65536 1272 / 492.  Columns in whole 16-byte chunks; sizes that the kernel's entry takes."""
+    65536 1272 / 492.  A bf16 weight (not ``wide``), whose library product needs no cast, from 768
+    rows on (64x64 over 300 rows 9.2 / 6.9, over 512 7.8 / 7.5, 192x64 over 777 9.1 / 15.5).  No side
+    below 32, a quarter of the kernel's tile (65536x8 over 8192 rows 1327 / 180, 24x8 over 1024 7.4 /
+    7.1).  Columns in whole 16-byte chunks; rows that the kernel's entry takes."""
     mn = out_features * in_features
-    return (out_features % 8 == 0 and in_features % 8 == 0 and mn <= 128 * rows and mn <= 1 << 20
-            and max(out_features, in_features) <= 65536 and rows < 1 << 30)
+    return (out_features % 8 == 0 and in_features % 8 == 0 and min(out_features, in_features) >= 32
+            and mn <= 128 * rows and mn <= 1 << 20 and (wide or rows >= 768) and rows < 1 << 30)
 
 
 def project(lin: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
@@ -122,7 +125,8 @@ def project(lin: torch.nn.Module, x: torch.Tensor) -> torch.Tensor:
     if (not bf16 or hooks or type(w) not in PLAIN or type(x) not in PLAIN or x.dim() < 2
             or x.shape[-1] != w.shape[1] or w.device != x.device
             or torch._C._functorch.peek_interpreter_stack() is not None
-            or not split_wgrad_applies(x.numel() // max(1, x.shape[-1]), *w.shape)):
+            or not split_wgrad_applies(x.numel() // max(1, x.shape[-1]), *w.shape,
+                                       w.dtype == torch.float32)):
         return lin(x)
     return torch.ops.pnfx.linear.default(x.to(torch.bfloat16), w)
 

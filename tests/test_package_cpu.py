@@ -239,19 +239,22 @@ def test_linear_op_gradients_are_those_of_the_library_linear(wdtype):
 
 
 def test_weight_gradient_rule_keeps_to_the_sizes_of_its_kernel():
-    """split_wgrad_applies sends nothing to pnfx_linear_wgrad that its entry refuses: up to 65536
-    features either way and fewer than 2^30 rows."""
+    """split_wgrad_applies sends nothing to pnfx_linear_wgrad that its entry refuses (over 65536 features,
+    2^30 rows), no thin weight, and few rows only where the library's product needs a cast."""
     from paper_01_anti_decoy_pnfirtau_amd.hip_pnfirtau import split_wgrad_applies
 
     lib = _lib.lib()
-    for rows, out, inp in [(8192, 131072, 8), (8192, 8, 131072), (8192, 65536, 16), (1 << 30, 8, 8),
-                           ((1 << 30) - 1, 8, 8), (16384, 768, 256)]:
-        fits = max(out, inp) <= 65536 and rows < 1 << 30
-        assert split_wgrad_applies(rows, out, inp) == fits
-        if not fits:  # refused on the host, before any device call
-            fake = ctypes.c_void_p(256)
-            assert lib.pnfx_linear_wgrad(fake, out, fake, inp, fake, out, inp, rows, _lib.PNFX_F32,
-                                         fake, 1 << 50, None) == -1
+    fake = ctypes.c_void_p(256)
+    for rows, out, inp in [(8192, 131072, 8), (8192, 8, 131072), (1 << 30, 64, 64)]:
+        assert not split_wgrad_applies(rows, out, inp)
+        # refused on the host, before any device call
+        assert lib.pnfx_linear_wgrad(fake, out, fake, inp, fake, out, inp, rows, _lib.PNFX_F32, fake,
+                                     1 << 50, None) == -1
+    for rows, out, inp, wide, fits in [(8192, 65536, 16, True, False), (8192, 32768, 32, True, True),
+                                       (16384, 768, 256, True, True), (16384, 768, 256, False, True),
+                                       (500, 192, 64, True, True), (500, 192, 64, False, False),
+                                       (768, 192, 64, False, True), (1024, 24, 8, True, False)]:
+        assert split_wgrad_applies(rows, out, inp, wide) == fits, (rows, out, inp, wide)
 
 
 def test_wikilm_variants_share_init_and_train_on_cpu():
