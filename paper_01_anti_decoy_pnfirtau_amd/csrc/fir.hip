@@ -69,18 +69,24 @@ struct FirArgs {
   const void* x;
   int64_t sb, sh, sn;
   void* y;
-  int64_t ysb, ysh, ysn;
   int64_t B, H, N, C;
   const float* taps;
   int64_t taps_rows;
   int K;
 };
+// Output rows of strides given.  A kernel of its own, with arguments of its own, writes them: the
+// strides and their arithmetic cost the contiguous calls up to 5 % (B=8 H=8 N=2048 d=64 bf16 5.8 -> 6.1 us).
+struct FirIntoArgs : FirArgs {
+  int64_t ysb, ysh, ysn;
+};
+template <bool INTO>
+using fir_args_t = std::conditional_t<INTO, FirIntoArgs, FirArgs>;
 
 // KT is the compile-time bound on the tap count (K <= KT); KT == 7 is the pn_fir_tau case.
 // grid.x covers the (run, chunk) pairs of one (b, h) slice, grid.y = b * H + h; all index
 // arithmetic except the final address is 32-bit (sizes are checked on the host).
-template <typename T, int KT, bool ADJ>
-__global__ __launch_bounds__(256) void fir_vec_kernel(FirArgs a) {
+template <typename T, int KT, bool ADJ, bool INTO>
+__global__ __launch_bounds__(256) void fir_vec_kernel(fir_args_t<INTO> a) {
   constexpr int VEC = Chunk<T>::VEC;
   constexpr int WIN = RUN + KT - 1;
   const int CH = (int)a.C / VEC;
@@ -116,8 +122,14 @@ __global__ __launch_bounds__(256) void fir_vec_kernel(FirArgs a) {
       win[w] = u32x4{0u, 0u, 0u, 0u};
     }
   }
-  T* ys = reinterpret_cast<T*>(a.y) + (int64_t)b * a.ysb + (int64_t)hh * a.ysh +
-          (int64_t)n0 * a.ysn + ch * VEC;
+  int64_t ysn = a.C;
+  T* ys = reinterpret_cast<T*>(a.y) + ch * VEC;
+  if constexpr (INTO) {
+    ysn = a.ysn;
+    ys += (int64_t)b * a.ysb + (int64_t)hh * a.ysh + n0 * ysn;
+  } else {
+    ys += ((int64_t)bh * N + n0) * a.C;
+  }
   // Window rows in the order of increasing lag (newest first for the forward, oldest first
   // for the adjoint): each row is widened to fp32 once and feeds every output of the run
   // that uses it, as that output's next term.  Output j (row n = n0 + j) sits at window
@@ -157,12 +169,12 @@ __global__ __launch_bounds__(256) void fir_vec_kernel(FirArgs a) {
   else chain(std::integral_constant<bool, true>{});
 #pragma unroll
   for (int j = 0; j < RUN; ++j)
-    if (n0 + j < N) store_chunk<T>(ys + (int64_t)j * a.ysn, acc[j]);
+    if (n0 + j < N) store_chunk<T>(ys + (int64_t)j * ysn, acc[j]);
 }
 
 // One thread per output element; any channel stride / alignment.
-template <typename T, bool ADJ>
-__global__ __launch_bounds__(256) void fir_scalar_kernel(FirArgs a, int64_t sc) {
+template <typename T, bool ADJ, bool INTO>
+__global__ __launch_bounds__(256) void fir_scalar_kernel(fir_args_t<INTO> a, int64_t sc) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= a.B * a.H * a.N * a.C) return;
   const int64_t c = t % a.C;
@@ -177,29 +189,38 @@ __global__ __launch_bounds__(256) void fir_scalar_kernel(FirArgs a, int64_t sc) 
     if (m < 0 || m >= a.N) break;
     acc = __builtin_fmaf(to_f32(xs[m * a.sn]), tp[a.K - 1 - u], acc);
   }
-  reinterpret_cast<T*>(a.y)[b * a.ysb + hh * a.ysh + n * a.ysn + c] = from_f32<T>(acc);
+  int64_t to = (bh * a.N + n) * a.C + c;
+  if constexpr (INTO) to = b * a.ysb + hh * a.ysh + n * a.ysn + c;
+  reinterpret_cast<T*>(a.y)[to] = from_f32<T>(acc);
 }
 
-template <typename T, bool ADJ>
-int launch_fir(const FirArgs& a, hipStream_t st) {
+template <typename T, bool ADJ, bool INTO>
+int launch_fir_to(const fir_args_t<INTO>& a, hipStream_t st) {
   constexpr int VEC = Chunk<T>::VEC;
-  const bool vec_ok = (reinterpret_cast<uintptr_t>(a.x) % 16 == 0) &&
-                      (reinterpret_cast<uintptr_t>(a.y) % 16 == 0) && a.C % VEC == 0 &&
-                      a.sb % VEC == 0 && a.sh % VEC == 0 && a.sn % VEC == 0 &&
-                      a.ysb % VEC == 0 && a.ysh % VEC == 0 && a.ysn % VEC == 0;
+  bool vec_ok = (reinterpret_cast<uintptr_t>(a.x) % 16 == 0) &&
+                (reinterpret_cast<uintptr_t>(a.y) % 16 == 0) && a.C % VEC == 0 &&
+                a.sb % VEC == 0 && a.sh % VEC == 0 && a.sn % VEC == 0;
+  if constexpr (INTO) vec_ok = vec_ok && a.ysb % VEC == 0 && a.ysh % VEC == 0 && a.ysn % VEC == 0;
   const int64_t per_slice = ((a.N + RUN - 1) / RUN) * (a.C / VEC);
   if (vec_ok && per_slice < (1ll << 30) && a.B * a.H < 65536 && a.N < (1ll << 30)) {
     const dim3 grid((unsigned)((per_slice + 255) / 256), (unsigned)(a.B * a.H));
     if (a.K == 7)
-      hipLaunchKernelGGL((fir_vec_kernel<T, 7, ADJ>), grid, dim3(256), 0, st, a);
+      hipLaunchKernelGGL((fir_vec_kernel<T, 7, ADJ, INTO>), grid, dim3(256), 0, st, a);
     else
-      hipLaunchKernelGGL((fir_vec_kernel<T, KMAX, ADJ>), grid, dim3(256), 0, st, a);
+      hipLaunchKernelGGL((fir_vec_kernel<T, KMAX, ADJ, INTO>), grid, dim3(256), 0, st, a);
   } else {
     const int64_t total = a.B * a.H * a.N * a.C;
-    hipLaunchKernelGGL((fir_scalar_kernel<T, ADJ>), dim3((total + 255) / 256), dim3(256), 0, st,
+    hipLaunchKernelGGL((fir_scalar_kernel<T, ADJ, INTO>), dim3((total + 255) / 256), dim3(256), 0, st,
                        a, (int64_t)1);
   }
   return launch_status(ADJ ? "pnfx_fir_bwd" : "pnfx_fir_fwd");
+}
+
+template <typename T>
+int launch_fir(bool adj, const FirIntoArgs& a, hipStream_t st) {
+  if (!adj) return launch_fir_to<T, false, false>(a, st);  // (its output is always contiguous)
+  const bool into = a.ysn != a.C || a.ysh != a.N * a.C || a.ysb != a.H * a.N * a.C;
+  return into ? launch_fir_to<T, true, true>(a, st) : launch_fir_to<T, true, false>(a, st);
 }
 
 int fir_entry(bool adj, const void* x, int64_t sb, int64_t sh, int64_t sn, void* y, int64_t ysb,
@@ -212,10 +233,10 @@ int fir_entry(bool adj, const void* x, int64_t sb, int64_t sh, int64_t sn, void*
   PNFX_REQUIRE(taps_rows == 1 || taps_rows == H, "fir: taps_rows=%lld must be 1 or H=%lld",
                (long long)taps_rows, (long long)H);
   if (B * H * N * C == 0) return PNFX_OK;
-  FirArgs a{x, sb, sh, sn, y, ysb, ysh, ysn, B, H, N, C, taps, taps_rows, K};
+  const FirIntoArgs a{{x, sb, sh, sn, y, B, H, N, C, taps, taps_rows, K}, ysb, ysh, ysn};
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (dtype == PNFX_BF16) return adj ? launch_fir<bf16, true>(a, st) : launch_fir<bf16, false>(a, st);
-  if (dtype == PNFX_F32) return adj ? launch_fir<float, true>(a, st) : launch_fir<float, false>(a, st);
+  if (dtype == PNFX_BF16) return launch_fir<bf16>(adj, a, st);
+  if (dtype == PNFX_F32) return launch_fir<float>(adj, a, st);
   set_error("fir: unsupported dtype %d", dtype);
   return PNFX_EUNSUPPORTED;
 }
