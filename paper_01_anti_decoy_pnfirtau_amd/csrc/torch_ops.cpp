@@ -12,6 +12,9 @@
 // pnfx::pn_rows_fwd / _bwd  _TritonPnFirTauScoresFn     :694-785
 // pnfx::flash_fwd / _bwd    _FlashPnFirTauFn            :814-968
 // pnfx::flash_fwd_fir       (none: the FIR fused into the forward's key-tile load)
+// pnfx::attn_rows / _bwd    (none: key FIR and flash on projection rows, one autograd node)
+// pnfx::linear / _wgrad     (none: x W^T with its weight gradient's fp32 sums)
+// pnfx::sum_f64             the fp64 sum of tau's row gradients  :784
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>

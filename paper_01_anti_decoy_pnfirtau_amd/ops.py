@@ -13,6 +13,10 @@ pnfx::fir_fwd / _bwd   _TritonCausalFir7Fn              :629-682
 pnfx::pn_rows_fwd/_bwd _TritonPnFirTauScoresFn          :694-785
 pnfx::flash_fwd/_bwd   _FlashPnFirTauFn                 :814-968
 pnfx::flash_fwd_fir    (none: the key FIR fused into the forward's key-tile load)
+pnfx::attn_rows/_bwd   (none: key FIR and flash on projection rows [B, N, 3 D], one autograd node)
+pnfx::linear           (none: x W^T whose weight gradient is linear_wgrad)
+pnfx::linear_wgrad     (none: dY^T X of bf16 rows, fp32 sums)
+pnfx::sum_f64          the fp64 sum of tau's row gradients  :784
 """
 from __future__ import annotations
 
