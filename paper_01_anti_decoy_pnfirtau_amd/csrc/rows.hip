@@ -10,7 +10,7 @@
 //
 // Bound: HBM for the bytes (the causal half of the inputs read, the whole output written), with
 // the vector units close behind: about 19 operations per entry forward and 27 backward.  On the
-// scores of [32, 4, 512, 512] bf16: forward 27.0 -> 25.8 us, backward 43.0 -> 33.5 us (per-entry 64-bit
+// scores of [32, 4, 512, 512] bf16: forward 27.0 -> 26.2 us, backward 43.0 -> 32.6 us (per-entry 64-bit
 // range tests and, in the backward, a division per entry before); [4, 8, 777, 777]: 23.8 -> 17.2 and
 // 34.0 -> 23.3 us (single elements per lane, and every chunk that a register could hold computed
 // whether or not the row reaches it, before).
